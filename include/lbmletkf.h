@@ -51,8 +51,8 @@ extern "C" {
 #define LBMLETKF_CLOSURE_MLP         1
 
 /* analysis variants */
-#define LBMLETKF_VARIANT_PLAIN       0   /* per-member LBM launches, FP32 Gram on VALU, FP64 Jacobi */
-#define LBMLETKF_VARIANT_MIXED       1   /* batched LBM + fused LETKF, mixed precision */
+#define LBMLETKF_VARIANT_PLAIN       0   /* FP32 Gram on VALU, FP64 Jacobi */
+#define LBMLETKF_VARIANT_MIXED       1   /* fused LETKF, mixed precision; cycles replayed as graphs */
 
 /* All physical / numerical parameters of a run.  The reference fixes these at
  * compile time in src/config.h and the makefile macros
@@ -343,14 +343,15 @@ int lbmletkf_trainer_train(lbmletkf_trainer* tr, int batch, int steps, double lr
                            float* loss_history);
 
 /* ---- tuning ----------------------------------------------------------------------
- * Launch shapes of the MIXED variant: the shape of the fused LBM step --
- * lbm_tiles_per_block = k > 0: k tiles of 64 x 16 per workgroup; = -h: full-row
+ * Launch shapes: the shape of the LBM step --
+ * lbm_tiles_per_block = 1 (the default): the library's rule on the grid and ensemble
+ * size (blocks of 16 x 16 nodes taking four steps per launch, or the strips below with
+ * a height of its own); = k > 1: k tiles of 64 x 16 per workgroup; = -h: full-row
  * strips of h rows (h = 8, 16, 32; nx a multiple of 64 up to 1024, one thread per
  * column); = -(100 + h): full-row strips of h rows advanced two steps per launch
  * (h = 16, 32; nx a multiple of 64 up to 1024); = -(200 + h): three steps per
- * launch (h = 16, 32; nx a multiple of 64 up to 512).  The multi-step strips serve
- * flows without body force or friction (others take one step per launch) and are
- * bit-identical to single steps -- and the chain length of the analysis (gridpoints
+ * launch (h = 16, 32; nx a multiple of 64 up to 512); all shapes give the same bits --
+ * and the chain length of the analysis (gridpoints
  * of one column per wavefront, each warm-started from the previous one's
  * eigenvectors; the result changes by FP32 rounding).
  * No counterpart in the reference. */

@@ -417,38 +417,52 @@ int prof_collect(Ctx* c) {
     return LBMLETKF_OK;
 }
 
-// n LBM steps of all members (src/lbm.h:16-29 applied n times): stream-ordered
-// launches only, so a cycle can be captured into a graph.  Advances cur and step.
-int forecast_launches(Ctx* c, int n_steps) {
+// The kernels of n LBM steps of all members (src/lbm.h:16-29 applied n times), the
+// last steps of a launch shape that takes several taking what is left.  Advances cur;
+// `launches` counts the kernels.
+hipError_t step_launches(Ctx* c, int n_steps, long long& launches) {
     const bool mlp = c->cfg.closure_kind == LBMLETKF_CLOSURE_MLP;
-    if (mlp && !c->closure_ready) return fail(c, LBMLETKF_ERR_STATE, "closure_kind is MLP: call lbmletkf_set_closure first");
-    const bool fused = mlp || (c->cfg.variant == LBMLETKF_VARIANT_MIXED && lbm_fused_supported(c->nx, c->ny));
-    hipEvent_t ev = prof_begin(c);
-    // the two- and three-step strips take several steps per launch (no forcing: no
-    // per-step field); the last steps of a forecast take what is left
-    const int per_launch = (fused && !mlp) ? lbm_launch_steps(*c) : 1;
-    long long launches = 0;
-    for (int s = 0; s < n_steps;) {
-        const int k = std::min(per_launch, n_steps - s);
-        if (c->lp.has_force) HIP_TRY(c, launch_force_field(*c, s));
+    const int per_launch = mlp ? 1 : lbm_launch_steps(*c);
+    hipError_t e = hipSuccess;
+    int first = 0, formed = 0;  // force_xy holds the fields of steps [first, formed)
+    for (int s = 0; s < n_steps && e == hipSuccess;) {
+        int k = std::min(per_launch, n_steps - s);
+        if (c->lp.has_force) {
+            if (s == formed) {
+                const int n = std::min(c->force_steps, n_steps - s);
+                e = launch_force_field(*c, s, n);
+                if (e != hipSuccess) return e;
+                launches += 2;
+                first = s;
+                formed = s + n;
+            }
+            k = std::min(k, formed - s);
+        }
+        const float* force = c->force_xy + (long long)(s - first) * 2 * c->nodes;
         const float* fin = c->f[c->cur];
         float* fout = c->f[1 - c->cur];
-        if (mlp) {
-            HIP_TRY(c, launch_lbm_mlp(*c, fin, fout, 0, (c->nx / 64) * (c->ny / 16) * c->M, nullptr));
-            ++launches;
-        } else if (fused) {
-            HIP_TRY(c, launch_lbm_fused(*c, fin, fout, k));
-            ++launches;
-        } else {
-            for (int m = 0; m < c->M; ++m) HIP_TRY(c, launch_lbm_plain_member(*c, fin, fout, m));
-            launches += 3LL * c->M;
-        }
-        if (c->lp.has_force) ++launches;
+        e = mlp ? launch_lbm_mlp(*c, fin, fout, force, 0, (c->nx / 64) * (c->ny / 16) * c->M, nullptr)
+                : launch_lbm_fused(*c, fin, fout, k, force);
+        ++launches;
         c->cur = 1 - c->cur;
         s += k;
     }
-    if (n_steps > 0) HIP_TRY(c, launch_step_advance(*c, n_steps));
-    prof_end(c, PH_FORECAST, ev, launches + (n_steps > 0), (long long)n_steps * c->M * c->nodes);
+    if (e == hipSuccess && n_steps > 0) {
+        e = launch_step_advance(*c, n_steps);
+        ++launches;
+    }
+    return e;
+}
+
+// n LBM steps: stream-ordered launches only, so a cycle can be captured into a graph.
+// Advances cur and step.
+int forecast_launches(Ctx* c, int n_steps) {
+    if (c->cfg.closure_kind == LBMLETKF_CLOSURE_MLP && !c->closure_ready)
+        return fail(c, LBMLETKF_ERR_STATE, "closure_kind is MLP: call lbmletkf_set_closure first");
+    hipEvent_t ev = prof_begin(c);
+    long long launches = 0;
+    HIP_TRY(c, step_launches(c, n_steps, launches));
+    prof_end(c, PH_FORECAST, ev, launches, (long long)n_steps * c->M * c->nodes);
     c->step += n_steps;
     return LBMLETKF_OK;
 }
@@ -555,7 +569,7 @@ void Ctx::drop_graphs() {
 
 Ctx::~Ctx() {
     drop_graphs();
-    void* ptrs[] = {f[0], f[1], plain_ruv, plain_nus, force_xy, d_force, d_step, d_status,
+    void* ptrs[] = {f[0], f[1], force_xy, d_force_draws, d_force_table, d_force, d_step, d_status,
                     d_site_node, d_loc_ptr, d_loc_site, d_loc_w, d_obs_coef, d_yo, d_hx, d_hx1, d_dy,
                     d_dyo, d_gram, d_bvec, d_mix_u, d_mix_b, d_dump, d_red, d_truth, d_sweeps,
                     d_sweeps64, d_closure, d_site_map, d_ens_uv, d_ens_out};
@@ -712,10 +726,12 @@ int lbmletkf_create(const lbmletkf_config* cfg, int n_members, lbmletkf_ctx** ou
     const size_t fsz = size_t(c->M) * Q * c->nodes;
     CREATE_TRY(dalloc(&c->f[0], fsz));
     CREATE_TRY(dalloc(&c->f[1], fsz));
-    CREATE_TRY(dalloc(&c->plain_ruv, 3 * c->nodes));
-    CREATE_TRY(dalloc(&c->plain_nus, c->nodes));
-    CREATE_TRY(dalloc(&c->force_xy, 2 * c->nodes));
+    c->force_steps = c->lp.has_force ? force_batch(c->nx, c->ny) : 1;
+    CREATE_TRY(dalloc(&c->force_xy, size_t(c->force_steps) * 2 * c->nodes));
     CREATE_TRY(hipMemset(c->force_xy, 0, sizeof(float) * 2 * c->nodes));
+    CREATE_TRY(dalloc(&c->d_force_draws, size_t(c->force_steps) * MAX_FORCE_MODES));
+    CREATE_TRY(dalloc(&c->d_force_table, size_t(force_table_entries(*c))));
+    CREATE_TRY(launch_force_table(*c));
     CREATE_TRY(dalloc(&c->d_force, 1));
     CREATE_TRY(hipMemcpy(c->d_force, &c->force, sizeof(ForceTable), hipMemcpyHostToDevice));
     CREATE_TRY(dalloc(&c->d_step, 1));
@@ -1411,20 +1427,8 @@ int group_analysis_launches(Group* g) {
 // sum of the contexts' one-step launches.  A context with the learned closure steps
 // with the closure kernel, one step per launch, as it does on its own.
 int group_context_steps(Group* g, Ctx* c, int n_steps) {
-    const bool mlp = c->cfg.closure_kind == LBMLETKF_CLOSURE_MLP;
-    const int per_launch = mlp ? 1 : lbm_launch_steps(*c);
-    for (int s = 0; s < n_steps;) {
-        const int k = std::min(per_launch, n_steps - s);
-        if (c->lp.has_force) G_HIP(g, launch_force_field(*c, s));
-        if (mlp)
-            G_HIP(g, launch_lbm_mlp(*c, c->f[c->cur], c->f[1 - c->cur], 0, (c->nx / 64) * (c->ny / 16) * c->M,
-                                    nullptr));
-        else
-            G_HIP(g, launch_lbm_fused(*c, c->f[c->cur], c->f[1 - c->cur], k));
-        c->cur = 1 - c->cur;
-        s += k;
-    }
-    if (n_steps > 0) G_HIP(g, launch_step_advance(*c, n_steps));
+    long long launches = 0;
+    G_HIP(g, step_launches(c, n_steps, launches));
     c->step += n_steps;
     return LBMLETKF_OK;
 }
@@ -1759,8 +1763,8 @@ int lbmletkf_autotune(lbmletkf_ctx* ctx, const char* cache_path, char* report, i
     }
     c->drop_graphs();
     char buf[128];
-    // 1. row-band height of the fused LBM kernel: 1, 2 or 4 tiles of 64x16 per workgroup
-    //    (the step writes the idle half of the double buffer only)
+    // 1. shape of the LBM step: the library's rule (1), 2 or 4 tiles of 64x16 per workgroup,
+    //    or strips (the step writes the idle half of the double buffer only)
     int best_tpb = c->lbm_tiles_per_block;
     if (mixed && lbm_fused_supported(c->nx, c->ny)) {
         const long long tiles = (long long)(c->nx / 64) * (c->ny / 16) * c->M;
@@ -1776,7 +1780,7 @@ int lbmletkf_autotune(lbmletkf_ctx* ctx, const char* cache_path, char* report, i
             c->lbm_tiles_per_block = tpb;
             const int k = lbm_launch_steps(*c);  // time per step (a launch may take several)
             double us = 0;
-            if (int st = time_launches(c, 2, 10, [&] { return launch_lbm_fused(*c, c->f[c->cur], c->f[1 - c->cur], k); }, us))
+            if (int st = time_launches(c, 2, 10, [&] { return launch_lbm_fused(*c, c->f[c->cur], c->f[1 - c->cur], k, c->force_xy); }, us))
                 return st;
             us /= k;
             std::snprintf(buf, sizeof buf, " %d:%.1f", tpb, us);

@@ -519,16 +519,17 @@ void closure_weights_host(const float* P, const lbmletkf_config& cfg, ClosureWei
     w.nu_max = float(cfg.closure_nu_max);
 }
 
-hipError_t launch_lbm_mlp(Ctx& c, const float* fin, float* fout, int tile0, int n_tiles, float* nut_out) {
+hipError_t launch_lbm_mlp(Ctx& c, const float* fin, float* fout, const float* field, int tile0, int n_tiles,
+                          float* nut_out) {
     const int tiles_x = c.nx / MX, tiles = tiles_x * (c.ny / MY);
     if (!c.d_closure || c.nx % MX || c.ny % MY || tile0 < 0 || n_tiles < 1 || tile0 + n_tiles > tiles * c.M)
         return hipErrorInvalidValue;
     const bool force = c.lp.has_force || c.lp.fric_over_dt != 0.f;
     if (force)
-        k_lbm_mlp<true><<<n_tiles, MNT, 0, c.stream>>>(fin, fout, c.force_xy, c.lp, c.d_closure, tiles_x, tiles, tile0,
+        k_lbm_mlp<true><<<n_tiles, MNT, 0, c.stream>>>(fin, fout, field, c.lp, c.d_closure, tiles_x, tiles, tile0,
                                                       nut_out);
     else
-        k_lbm_mlp<false><<<n_tiles, MNT, 0, c.stream>>>(fin, fout, c.force_xy, c.lp, c.d_closure, tiles_x, tiles,
+        k_lbm_mlp<false><<<n_tiles, MNT, 0, c.stream>>>(fin, fout, field, c.lp, c.d_closure, tiles_x, tiles,
                                                        tile0, nut_out);
     return hipGetLastError();
 }
@@ -853,7 +854,7 @@ int lbmletkf_closure_nut(lbmletkf_ctx* ctx, int member, float* nut) {
     if (e != hipSuccess) return report_error(c, LBMLETKF_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
     // the populations go to the idle half of the double buffer, which the next step overwrites
     const int tiles = (c->nx / 64) * (c->ny / 16);
-    e = launch_lbm_mlp(*c, c->f[c->cur], c->f[1 - c->cur], member * tiles, tiles, d);
+    e = launch_lbm_mlp(*c, c->f[c->cur], c->f[1 - c->cur], c->force_xy, member * tiles, tiles, d);
     if (e == hipSuccess) e = hipMemcpyAsync(nut, d, sizeof(float) * c->nodes, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     (void)hipFree(d);

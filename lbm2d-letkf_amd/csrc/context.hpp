@@ -81,11 +81,13 @@ struct Ctx {
     // state, double-buffered SoA f[member][q][j][i]
     float* f[2] = {nullptr, nullptr};
     int cur = 0;
-    // plain-variant intermediates, one member at a time: rho,u,v after streaming, nu_t
-    float* plain_ruv = nullptr;   // [3][nodes]
-    float* plain_nus = nullptr;   // [nodes]
-    // forcing field of the current step, shared by all members: [2][nodes]
+    // forcing fields of the next force_steps steps, shared by all members:
+    // [force_steps][2][nodes], the modes' coefficients they are formed from, and the
+    // table of the phases' sines and cosines
     float* force_xy = nullptr;
+    float2* d_force_draws = nullptr;  // [force_steps][MAX_FORCE_MODES]
+    float2* d_force_table = nullptr;  // [force_table_entries]
+    int force_steps = 0;
     ForceTable* d_force = nullptr;
     long long* d_step = nullptr;  // device copy of the step counter (graph-replay safe)
     long long step = 0;
@@ -118,7 +120,8 @@ struct Ctx {
     float* d_mix_b = nullptr;     // [nodes][N] b = dY^T R^-1 dyo
     int mix_width = 0;
     int mix_chain = 8;            // consecutive gridpoints per wavefront in k_mixed_solve
-    // shape of the fused LBM step: k > 0 tiles of 64x16 per workgroup (k_lbm_fused),
+    // shape of the LBM step: 1 the rule of lbm.hip on the grid and ensemble size (blocks
+    // or strips), k > 1 tiles of 64x16 per workgroup (k_lbm_fused),
     // -h full-row strips of h rows (k_lbm_rows), -(LBM_TWO_STEP + h) full-row strips
     // of h rows advanced two steps per launch (k_lbm_rows2), -(LBM_THREE_STEP + h)
     // three steps per launch (k_lbm_rows3)
@@ -173,13 +176,20 @@ struct Ctx {
 int report_error(Ctx* c, int code, const std::string& msg);
 
 // ---- launchers (lbm.hip) ------------------------------------------------------
-hipError_t launch_force_field(Ctx& c, int step_offset);
-// one launch of the fused step in the tuned shape, advancing `steps` steps (up to
-// lbm_launch_steps(c))
-hipError_t launch_lbm_fused(Ctx& c, const float* fin, float* fout, int steps = 1);
-// steps one launch of the tuned shape can take without forcing: 3 for the
-// three-step strips (lbm_tiles_per_block <= -LBM_THREE_STEP), 2 for the two-step
-// strips (<= -LBM_TWO_STEP), else 1; 1 for any forced flow
+// the forcing fields of steps [step + step_offset, + steps) into force_xy, steps up to
+// force_steps
+hipError_t launch_force_field(Ctx& c, int step_offset, int steps);
+// steps whose forcing fields are formed by one launch at this grid size
+int force_batch(int nx, int ny);
+// the table of the forcing phases: its entries (0: none), and the kernel that fills it
+long long force_table_entries(const Ctx& c);
+hipError_t launch_force_table(Ctx& c);
+// one launch of the step in the context's shape, advancing all members by `steps`
+// steps (up to lbm_launch_steps(c)); force: the first of these steps' fields (unused
+// by flows without forcing)
+hipError_t launch_lbm_fused(Ctx& c, const float* fin, float* fout, int steps, const float* force);
+// steps one launch of the context's shape can take: 3 for the three-step strips, 2
+// for the two-step strips, else 1
 int lbm_launch_steps(const Ctx& c);
 // the MIXED analysis of several contexts (obs already prepared) in one launch of
 // each of its two kernels, on `stream`
@@ -187,8 +197,8 @@ hipError_t launch_letkf_mixed_group(Ctx* const* cs, int n, hipStream_t stream);
 // one step with the learned closure for tiles [tile0, tile0 + n_tiles) of the
 // 64x16 tiling (member-major); nut_out (may be NULL) receives nu_t of those
 // tiles' nodes, indexed by node within the member
-hipError_t launch_lbm_mlp(Ctx& c, const float* fin, float* fout, int tile0, int n_tiles, float* nut_out);
-hipError_t launch_lbm_plain_member(Ctx& c, const float* fin, float* fout, int member);
+hipError_t launch_lbm_mlp(Ctx& c, const float* fin, float* fout, const float* force, int tile0, int n_tiles,
+                          float* nut_out);
 hipError_t launch_nudge(Ctx& c, const float* ro, const float* uo, const float* vo, float alpha, int xyprune,
                         int skip_east, int skip_north, int use_obs_rho);
 hipError_t launch_perturb(Ctx& c, int member, const float* ur, const float* vr, float eps);

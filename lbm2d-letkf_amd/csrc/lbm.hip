@@ -6,16 +6,19 @@
 //   (src/lbm.cu:24-65) -> BGK relaxation with tau = 0.5 + 3(nu+nu_t)/(c^2 dt)
 //   and the first-order force term (src/lbm.cu:105-160, src/lbm.h:31-70).
 //
-// Two forms are built:
-//   * lbm_fused: one launch advances every member by one step.  A 64x16 tile of
+// One launch advances every member by one to three steps, in one of these shapes:
+//   * tiles: one step.  A 64x16 tile of
 //     one member is streamed into registers, its streamed velocity (plus a one-node
 //     halo) goes to LDS for the strain stencil, and the collided populations are
 //     written once: 36 B read + 36 B written per node update.  A workgroup may
 //     take several tiles of a row band in turn (one per workgroup is fastest at
-//     256^2 x 64: the tiles of one workgroup do not overlap their loads).
-//   * the plain form keeps the reference's three passes (stream+macro, les,
-//     collide) and is launched member by member, as one reference rank would.
+//     256^2 x 64: the tiles of one workgroup do not overlap their loads).  Any grid.
+//   * full-row strips, one thread per column: one, two or three steps.
+#include <algorithm>
+#include <climits>
+#include <cmath>
 #include <map>
+#include <numeric>
 #include <type_traits>
 #include <mutex>
 
@@ -37,8 +40,11 @@ constexpr int ROWS_PER_PASS = NT / TX;        // 4
 constexpr int NODES_PER_THREAD = TY / ROWS_PER_PASS;  // 4
 constexpr int HALO = 2 * (TX + 2) + 2 * TY;   // 164
 
-// Tile t (member-major order of 64x16 tiles) of one step.
-template <bool FORCE>
+// Tile t (member-major order of 64x16 tiles) of one step.  RAGGED: grids that are
+// not multiples of the tile; the columns and rows past the edge stream the periodic
+// image of their node (so that the stencil of the edge nodes finds its neighbours)
+// and write nothing.
+template <bool FORCE, bool RAGGED>
 __device__ __forceinline__ void lbm_tile(int t, const float* __restrict__ fin, float* __restrict__ fout,
                                          const float* __restrict__ force, const LbmParams& p, int tiles_x,
                                          int tiles_per_member) {
@@ -54,7 +60,7 @@ __device__ __forceinline__ void lbm_tile(int t, const float* __restrict__ fin, f
     const int y0 = (tt / tiles_x) * TY;
     const float* f = fin + (long long)member * p.member_stride;
     float* fo = fout + (long long)member * p.member_stride;
-    const int i = x0 + lx;
+    const int i = RAGGED ? (x0 + lx) % nx : x0 + lx;
     const int im = wrap(i - 1, nx), ip = wrap(i + 1, nx);
 
     __syncthreads();  // the previous tile's stencil reads of su/sv are done
@@ -63,7 +69,7 @@ __device__ __forceinline__ void lbm_tile(int t, const float* __restrict__ fin, f
 #pragma unroll
     for (int r = 0; r < NODES_PER_THREAD; ++r) {
         const int ly = ly0 + r * ROWS_PER_PASS;
-        const int j = y0 + ly;
+        const int j = RAGGED ? (y0 + ly) % ny : y0 + ly;
         const long long r0 = (long long)j * nx;
         const long long rm = (long long)wrap(j - 1, ny) * nx;
         const long long rp = (long long)wrap(j + 1, ny) * nx;
@@ -79,7 +85,8 @@ __device__ __forceinline__ void lbm_tile(int t, const float* __restrict__ fin, f
         else if (h < 2 * (TX + 2)) { hx = h - (TX + 2) - 1; hy = TY; }
         else if (h < 2 * (TX + 2) + TY) { hx = -1; hy = h - 2 * (TX + 2); }
         else { hx = TX; hy = h - 2 * (TX + 2) - TY; }
-        const int gi = wrap(x0 + hx, nx), gj = wrap(y0 + hy, ny);
+        const int gi = RAGGED ? (x0 + hx + nx) % nx : wrap(x0 + hx, nx);
+        const int gj = RAGGED ? (y0 + hy + ny) % ny : wrap(y0 + hy, ny);
         const int gim = wrap(gi - 1, nx), gip = wrap(gi + 1, nx);
         const long long r0 = (long long)gj * nx;
         const long long rm = (long long)wrap(gj - 1, ny) * nx;
@@ -95,6 +102,7 @@ __device__ __forceinline__ void lbm_tile(int t, const float* __restrict__ fin, f
     for (int r = 0; r < NODES_PER_THREAD; ++r) {
         const int ly = ly0 + r * ROWS_PER_PASS;
         const int j = y0 + ly;
+        if (RAGGED && (x0 + lx >= nx || j >= ny)) continue;
         const float nut = smagorinsky(su[ly + 1][lx + 2], su[ly + 1][lx], su[ly + 2][lx + 1],
                                       su[ly][lx + 1], sv[ly + 1][lx + 2], sv[ly + 1][lx],
                                       sv[ly + 2][lx + 1], sv[ly][lx + 1], p);
@@ -110,7 +118,7 @@ __device__ __forceinline__ void lbm_tile(int t, const float* __restrict__ fin, f
     }
 }
 
-template <bool FORCE>
+template <bool FORCE, bool RAGGED>
 __global__ __launch_bounds__(NT) void k_lbm_fused(const float* __restrict__ fin,
                                                   float* __restrict__ fout,
                                                   const float* __restrict__ force, LbmParams p,
@@ -123,7 +131,7 @@ __global__ __launch_bounds__(NT) void k_lbm_fused(const float* __restrict__ fin,
     const int b = blockIdx.x;
     const int bb = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
     for (int k = 0; k < tiles_per_block; ++k)
-        lbm_tile<FORCE>(bb * tiles_per_block + k, fin, fout, force, p, tiles_x, tiles_per_member);
+        lbm_tile<FORCE, RAGGED>(bb * tiles_per_block + k, fin, fout, force, p, tiles_x, tiles_per_member);
 }
 
 // Full-row strips: a workgroup of nx threads (one per column, nx a multiple of
@@ -192,9 +200,9 @@ __global__ __launch_bounds__(1024) void k_lbm_rows(const float* __restrict__ fin
     }
 }
 
-// Two steps per launch (no body force, no friction): a workgroup of nx threads
-// (one per column, nx <= 1024) produces rows [y0, y0+H) of one member at t+2 from
-// the populations at t; the intermediate step never leaves the chip.  Iteration k
+// Two steps per launch: a workgroup of nx threads (one per column, nx <= 1024; nx
+// rounded up to whole wavefronts, the lanes past the row writing nothing) produces
+// rows [y0, y0+H) of one member at t+2 from the populations at t; the intermediate step never leaves the chip.  Iteration k
 // runs four stages, each on another row and each followed by a barrier:
 //   A (row k):   pull from global (t), moments -> step-1 velocity ring u1/v1
 //   B (row k-1): Smagorinsky from u1/v1, collide -> populations at t+1 -> ring p1
@@ -213,9 +221,12 @@ __global__ __launch_bounds__(1024) void k_lbm_rows(const float* __restrict__ fin
 // written per node per launch, i.e. per two steps.
 constexpr int P1Q = 6;  // populations in the ring: q = 0, 2, 3, 5, 6, 8
 __device__ __forceinline__ constexpr int p1_slot(int q) { return (q / 3) * 2 + (q % 3 == 2 ? 1 : 0); }
-template <int H>
+// H = 0 takes the strip height `rows` at run time; the last strip of a member ends
+// at row ny.  FORCE: the body force of step s at force[s][2][nodes], and friction.
+template <int H, bool FORCE>
 __global__ __launch_bounds__(1024) void k_lbm_rows2(const float* __restrict__ fin, float* __restrict__ fout,
-                                                   LbmParams p, int strips_per_member) {
+                                                   const float* __restrict__ force, LbmParams p,
+                                                   int strips_per_member, int rows) {
     extern __shared__ float lds2[];  // u1, v1, u2, v2: [3][nx] each; p1: [3][P1Q][nx]
     const int nx = p.nx, ny = p.ny;
     const int nodes = int(p.nodes);  // offsets within one member fit in 32 bits
@@ -227,10 +238,12 @@ __global__ __launch_bounds__(1024) void k_lbm_rows2(const float* __restrict__ fi
     const int nb = gridDim.x, b = blockIdx.x;
     const int bb = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
     const int member = bb / strips_per_member;
-    const int y0 = (bb - member * strips_per_member) * H;
+    const int y0 = (bb - member * strips_per_member) * (H > 0 ? H : rows);
+    const int hs = H > 0 ? H : min(rows, ny - y0);
     const float* f = fin + (long long)member * p.member_stride;
     float* fo = fout + (long long)member * p.member_stride;
-    const int i = threadIdx.x;
+    const bool on = H > 0 || int(threadIdx.x) < nx;  // H > 0: rows of whole wavefronts
+    const int i = on ? threadIdx.x : nx - 1;
     const int im = i == 0 ? nx - 1 : i - 1, ip = i == nx - 1 ? 0 : i + 1;
     auto sl = [](int r) { return (r + 9) % 3; };  // ring slot of strip row r >= -9
     // unsigned 32-bit offsets from the member's base: the loads and stores address
@@ -249,6 +262,14 @@ __global__ __launch_bounds__(1024) void k_lbm_rows2(const float* __restrict__ fi
         fc[7] = f[7 * un + rm + ui];
         fc[8] = f[8 * un + rm + uim];
     };
+    // body force of step s at strip row r
+    auto force_at = [&](int s, int r, float& Fx, float& Fy) {
+        if (!FORCE || !p.has_force) return;
+        const unsigned node = unsigned(wrap(y0 + r, ny) * nx) + ui;
+        Fx = force[unsigned(2 * s) * un + node];
+        Fy = force[unsigned(2 * s + 1) * un + node];
+    };
+    float gx[2] = {0.f, 0.f}, gy[2] = {0.f, 0.f};  // requested an iteration ahead
     float q4m1 = 0.f, q7m1 = 0.f, q7m2 = 0.f;  // f1[4] of row k-2, f1[7] of rows k-2, k-3
     float fP[Q];
     // One iteration.  A writes (fa, ma) for row k; B reads the previous A row (fb,
@@ -260,22 +281,27 @@ __global__ __launch_bounds__(1024) void k_lbm_rows2(const float* __restrict__ fi
         // A: row k (the pull was issued one iteration earlier)
 #pragma unroll
         for (int q = 0; q < Q; ++q) fa[q] = fP[q];
-        if (k < H + 2) pull_g(k + 1, fP);
+        if (k < hs + 2) pull_g(k + 1, fP);
         moments(fa, p.c, ma[0], ma[1], ma[2]);
-        u1[sl(k) * nx + i] = ma[1];
-        v1[sl(k) * nx + i] = ma[2];
+        if (on) {
+            u1[sl(k) * nx + i] = ma[1];
+            v1[sl(k) * nx + i] = ma[2];
+        }
         __syncthreads();
         // B: row k-1, the populations at t+1
         if (k >= -1) {
             const int s = sl(k - 1) * nx, sn = sl(k) * nx, ss = sl(k - 2) * nx;
             const float nut = smagorinsky(u1[s + ip], u1[s + im], u1[sn + i], u1[ss + i], v1[s + ip],
                                           v1[s + im], v1[sn + i], v1[ss + i], p);
-            collide9<false>(fb, mb[0], mb[1], mb[2], nut, 0.f, 0.f, p);
+            collide9<FORCE>(fb, mb[0], mb[1], mb[2], nut, gx[0], gy[0], p);
             float* pr = p1 + sl(k - 1) * P1Q * nx;
+            if (on) {
 #pragma unroll
-            for (int q = 0; q < Q; ++q)
-                if (q % 3 != 1) pr[p1_slot(q) * nx + i] = fb[q];
+                for (int q = 0; q < Q; ++q)
+                    if (q % 3 != 1) pr[p1_slot(q) * nx + i] = fb[q];
+            }
         }
+        if (k >= -2) force_at(0, k, gx[0], gy[0]);
         __syncthreads();
         // C: row k-2, pulled from the ring (row above = k-1, below = k-3) and, for
         // q = 1, 4, 7, from this thread's own rows
@@ -293,37 +319,43 @@ __global__ __launch_bounds__(1024) void k_lbm_rows2(const float* __restrict__ fi
             fc[7] = q7m2;
             fc[8] = pm[p1_slot(8) * nx + im];
             moments(fc, p.c, mc[0], mc[1], mc[2]);
-            u2[sl(k - 2) * nx + i] = mc[1];
-            v2[sl(k - 2) * nx + i] = mc[2];
+            if (on) {
+                u2[sl(k - 2) * nx + i] = mc[1];
+                v2[sl(k - 2) * nx + i] = mc[2];
+            }
         }
         q7m2 = q7m1;
         q7m1 = fb[7];
         q4m1 = fb[4];
         __syncthreads();
         // D: row k-3, the populations at t+2
-        if (k >= 3) {
+        if (k >= 3 && k - 3 < hs) {
             const int s = sl(k - 3) * nx, sn = sl(k - 2) * nx, ss = sl(k - 4) * nx;
             const float nut = smagorinsky(u2[s + ip], u2[s + im], u2[sn + i], u2[ss + i], v2[s + ip],
                                           v2[s + im], v2[sn + i], v2[ss + i], p);
-            collide9<false>(fd, md[0], md[1], md[2], nut, 0.f, 0.f, p);
+            collide9<FORCE>(fd, md[0], md[1], md[2], nut, gx[1], gy[1], p);
             const unsigned node = unsigned((y0 + k - 3) * nx) + ui;
+            if (on) {
 #pragma unroll
-            for (int q = 0; q < Q; ++q) fo[unsigned(q) * un + node] = fd[q];
+                for (int q = 0; q < Q; ++q) fo[unsigned(q) * un + node] = fd[q];
+            }
         }
+        if (k >= 2) force_at(1, k - 2, gx[1], gy[1]);
     };
     float fX[Q], fY[Q], fZ[Q], fW[Q], mX[3], mY[3] = {0.f, 0.f, 0.f}, mZ[3], mW[3] = {0.f, 0.f, 0.f};
 #pragma unroll
     for (int q = 0; q < Q; ++q) fY[q] = fW[q] = 0.f;
     pull_g(-3, fP);
-    static_assert((H + 6) % 2 == 0, "iterations come in pairs");
-    for (int k = -3; k <= H + 2; k += 2) {
+    // iterations come in pairs: with an odd height the last one runs past the strip
+    // and writes nothing
+    for (int k = -3; k <= hs + 2; k += 2) {
         iter(k, fX, mX, fY, mY, fZ, mZ, fW, mW);
         iter(k + 1, fY, mY, fX, mX, fW, mW, fZ, mZ);
     }
 }
 
-// Three steps per launch (no body force, no friction), the two-step pipeline
-// extended by two stages: iteration k runs six stages a row apart:
+// Three steps per launch, the two-step pipeline extended by two stages: iteration k
+// runs six stages a row apart:
 //   A (row k):   pull from global (t), moments -> velocity ring 1
 //   B (row k-1): Smagorinsky, collide -> populations at t+1 -> population ring 1
 //   C (row k-2): pull from population ring 1, moments -> velocity ring 2
@@ -357,7 +389,10 @@ struct PopRing {
     float* q68;  // [3][2][nx]  q = 6, 8 of rows r mod 3
 };
 // NX > 0: the row length as a compile-time constant (every LDS ring offset then
-// becomes an immediate of its instruction); NX = 0 takes p.nx.
+// becomes an immediate of its instruction); NX = 0 takes p.nx.  H = 0 takes the strip
+// height `rows` at run time, the last strip of a member ending at row ny, and any
+// row length (nx rounded up to whole wavefronts, the lanes past the row writing
+// nothing).  FORCE: the body force of step s at force[s][2][nodes], and friction.
 // Odd strips are stepped as the lattice reflected in y: logical row r is physical
 // row y0 + H - 1 - r, and population q is the physical population with e_y
 // negated (0, 1, 2 <-> 6, 7, 8), so those strips walk their rows bottom-up.  The
@@ -366,9 +401,10 @@ struct PopRing {
 // population offsets of the loads and stores.  Two neighbouring strips then reach
 // their common boundary rows together (at the start of both, or at the end of
 // both), and the second read of those halo rows finds them in L2.
-template <int H, int NX>
+template <int H, int NX, bool FORCE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_lbm_rows3(
-    const float* __restrict__ fin, float* __restrict__ fout, LbmParams p, int strips_per_member) {
+    const float* __restrict__ fin, float* __restrict__ fout, const float* __restrict__ force, LbmParams p,
+    int strips_per_member, int rows) {
     extern __shared__ float lds3[];  // velocity rings [3 stages][u, v][2][nx]; population rings [2][12][nx]
     const int nx = NX > 0 ? NX : p.nx, ny = p.ny;
     const int nodes = int(p.nodes);  // offsets within one member fit in 32 bits
@@ -379,7 +415,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     const int bb = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
     const int member = bb / strips_per_member;
     const int strip = bb - member * strips_per_member;
-    const int y0 = strip * H;
+    const int y0 = strip * (H > 0 ? H : rows);
+    const int hs = H > 0 ? H : min(rows, ny - y0);
     const bool mir = (strip & 1) != 0;  // uniform
     // the member's populations through buffer resources: the byte offset of
     // population q in row j, (q nodes + j nx) 4, is uniform and goes to the scalar
@@ -390,7 +427,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         const_cast<float*>(fin + (long long)member * p.member_stride), 0, Q * nodes * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t fw =
         __builtin_amdgcn_make_buffer_rsrc(fout + (long long)member * p.member_stride, 0, Q * nodes * 4, 0x00020000);
-    const int i = threadIdx.x;
+    const bool on = H > 0 || int(threadIdx.x) < nx;  // H > 0: rows of whole wavefronts
+    const int i = on ? threadIdx.x : nx - 1;
     const int im = i == 0 ? nx - 1 : i - 1, ip = i == nx - 1 ? 0 : i + 1;
     const int bi = 4 * i, bim = 4 * im, bip = 4 * ip;
     auto ld = [&](int voff, int soff) {
@@ -398,7 +436,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     };
     // pull of logical row r: fc[q] = f[q](i - ex_q, r - ey_q) of the (reflected) lattice
     auto pull_g = [&](int r, float (&fc)[Q]) {
-        const int j = wrap(mir ? y0 + H - 1 - r : y0 + r, ny);
+        const int j = wrap(mir ? y0 + hs - 1 - r : y0 + r, ny);
         const int rm = 4 * wrap(j - 1, ny) * nx, r0 = 4 * j * nx, rp = 4 * wrap(j + 1, ny) * nx;
         const int qn = 4 * nodes;
         // physical offsets of logical population 0 (pulled from logical row r + 1) and
@@ -414,6 +452,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         fc[7] = ld(bi, on + qn);
         fc[8] = ld(bim, on + 2 * qn);
     };
+    // body force of step s at logical row r; the reflection turns its y component
+    const __amdgpu_buffer_rsrc_t rforce = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(force), 0, FORCE && p.has_force ? 6 * nodes * 4 : 0, 0x00020000);
+    auto force_at = [&](int s, int r, float& Fx, float& Fy) {
+        if (!FORCE || !p.has_force) return;
+        const int row = 4 * wrap(mir ? y0 + hs - 1 - r : y0 + r, ny) * nx + 8 * s * nodes;
+        Fx = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rforce, bi, row, 0));
+        Fy = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rforce, bi, row + 4 * nodes, 0));
+    };
+    // the force each collide stage takes next: requested as soon as the stage has used
+    // the last one, an iteration ahead
+    float gx[3] = {0.f, 0.f, 0.f}, gy[3] = {0.f, 0.f, 0.f};
     // LDS column offsets of this thread and its west and east neighbours, renewed
     // from an opaque copy at every iteration: formed once outside the loop, the
     // ring addresses built on them would stay live across it and spill
@@ -436,6 +486,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         fc[8] = d[nx + cm];
     };
     auto to_ring = [&](const PopRing& R, int r, const float (&fd)[Q]) {
+        if (!on) return;
         R.q02[ci] = fd[0];
         R.q02[nx + ci] = fd[2];
         float* c = q35_slot(R, r);
@@ -448,6 +499,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     // velocity ring of stage s (0, 1, 2): u of row r at vel[(s * 4 + (r & 1)) * nx],
     // v two slots further
     auto vel_put = [&](int s, int r, float u, float v) {
+        if (!on) return;
         vel[(s * 4 + (r & 1)) * nx + ci] = u;
         vel[(s * 4 + 2 + (r & 1)) * nx + ci] = v;
     };
@@ -458,7 +510,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         const float* ur = vel + (s * 4 + (r & 1)) * nx;
         const float* vr = vel + (s * 4 + 2 + (r & 1)) * nx;
         const float nut = smagorinsky(ur[cp], ur[cm], uN, uS, vr[cp], vr[cm], vN, vS, p);
-        collide9<false>(fd, md[0], md[1], md[2], nut, 0.f, 0.f, p);
+        collide9<FORCE>(fd, md[0], md[1], md[2], nut, gx[s], mir ? -gy[s] : gy[s], p);
     };
     // e_x = 0 populations of the collided rows: q4 of the last row, q7 of the last two
     float a4m1 = 0.f, a7m1 = 0.f, a7m2 = 0.f;  // step one
@@ -485,7 +537,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         float (&fP)[Q] = decltype(parity)::value ? fP1 : fP0;
 #pragma unroll
         for (int q = 0; q < Q; ++q) fa[q] = fP[q];
-        if (k + 2 <= H + 4) pull_g(k + 2, fP);
+        if (k + 2 <= hs + 4) pull_g(k + 2, fP);
         moments(fa, p.c, ma[0], ma[1], ma[2]);
         vel_put(0, k, ma[1], ma[2]);
         __builtin_amdgcn_sched_barrier(0);  // stages stay in order (register pressure)
@@ -494,6 +546,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
             collide_row(0, k - 1, ma[1], ma[2], uSa, vSa, fb, mb);
             to_ring(r1, k - 1, fb);
         }
+        if (k >= -4) force_at(0, k, gx[0], gy[0]);
         __syncthreads();
         // C: row k-2 at t+1
         const float uSc = mc[1], vSc = mc[2];
@@ -511,6 +564,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
             collide_row(1, k - 3, mc[1], mc[2], uSc, vSc, fd, md);
             to_ring(r2, k - 3, fd);
         }
+        if (k >= 0) force_at(1, k - 2, gx[1], gy[1]);
         __syncthreads();
         // E: row k-4 at t+2
         const float uSe = me[1], vSe = me[2];
@@ -524,17 +578,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         b4m1 = fd[4];
         __builtin_amdgcn_sched_barrier(0);
         // F: row k-5 -> populations at t+3, written out
-        if (k >= 5) {
+        if (k >= 5 && k - 5 < hs) {
             collide_row(2, k - 5, me[1], me[2], uSe, vSe, ff, mf);
-            const int row = 4 * (mir ? y0 + H - 1 - (k - 5) : y0 + k - 5) * nx;
+            const int row = 4 * (mir ? y0 + hs - 1 - (k - 5) : y0 + k - 5) * nx;
             // physical offsets of logical populations 0 and 6 (the reflection swaps them)
             const int o0 = (mir ? 24 : 0) * nodes + row, o6 = (mir ? 0 : 24) * nodes + row;
+            if (on) {
 #pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                const int off = q < 3 ? o0 + 4 * q * nodes : (q < 6 ? 4 * q * nodes + row : o6 + 4 * (q - 6) * nodes);
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, ff[q]), fw, bi, off, 0);
+                for (int q = 0; q < Q; ++q) {
+                    const int off = q < 3 ? o0 + 4 * q * nodes
+                                          : (q < 6 ? 4 * q * nodes + row : o6 + 4 * (q - 6) * nodes);
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, ff[q]), fw, bi, off, 0);
+                }
             }
         }
+        if (k >= 4) force_at(2, k - 4, gx[2], gy[2]);
     };
     float fX[Q], fY[Q], fZ[Q], fW[Q], fS[Q], fT[Q];
     float mX[3] = {0.f, 0.f, 0.f}, mY[3] = {0.f, 0.f, 0.f}, mZ[3] = {0.f, 0.f, 0.f}, mW[3] = {0.f, 0.f, 0.f},
@@ -543,64 +601,82 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     for (int q = 0; q < Q; ++q) fY[q] = fW[q] = fT[q] = 0.f;
     pull_g(-5, fP1);
     pull_g(-4, fP0);
-    static_assert((H + 10) % 2 == 0, "iterations come in pairs");
-    for (int k = -5; k <= H + 4; k += 2) {  // k odd
+    // iterations come in pairs: with an odd height the last one runs past the strip
+    // and writes nothing
+    for (int k = -5; k <= hs + 4; k += 2) {  // k odd
         iter(std::integral_constant<int, 1>{}, k, fX, mX, fY, mY, fZ, mZ, fW, mW, fS, mS, fT, mT);
         iter(std::integral_constant<int, 0>{}, k + 1, fY, mY, fX, mX, fW, mW, fZ, mZ, fT, mT, fS, mS);
     }
 }
 
 
-
-// ----------------------------------------------------------------------------
-// plain form: the reference's three passes for one member
-// ----------------------------------------------------------------------------
-__global__ void k_stream_macro(const float* __restrict__ f, float* __restrict__ fn,
-                               float* __restrict__ ruv, LbmParams p) {
-    const long long node = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (node >= p.nodes) return;
+// Up to four steps per launch of a 16x16 block of nodes, for problems too small to
+// fill the chip with strips: a workgroup holds the block and its halo (two nodes per
+// step and side: one for the pull, one for the central differences) as 32x32 nodes,
+// one per thread, and steps them in LDS, the region that is still exact shrinking by
+// two nodes per side and step.  The first pull reads global memory, the last collide
+// writes it.  Any grid: region nodes outside the grid are periodic images.
+// Latency bounds it (one 256^2 member: 1.9 us per step against 5.2 in one-step tiles, a
+// launch of which costs as much however little it does); four steps take 16 + 16 nodes a
+// side, the most that one thread per node allows.
+constexpr int BL = 16, BL_STEPS = 4, BL_R = BL + 4 * BL_STEPS;
+template <bool FORCE>
+__global__ __launch_bounds__(BL_R * BL_R) void k_lbm_block(const float* __restrict__ fin, float* __restrict__ fout,
+                                                          const float* __restrict__ force, LbmParams p,
+                                                          int blocks_x, int blocks_per_member, int steps) {
+    __shared__ float fs[Q][BL_R * BL_R];
+    __shared__ float su[BL_R * BL_R], sv[BL_R * BL_R];
     const int nx = p.nx, ny = p.ny;
-    const int i = int(node % nx), j = int(node / nx);
-    float fc[Q];
-    pull9(f, p.nodes, wrap(i - 1, nx), i, wrap(i + 1, nx), (long long)wrap(j - 1, ny) * nx,
-          (long long)j * nx, (long long)wrap(j + 1, ny) * nx, fc);
+    const long long nodes = p.nodes;
+    const int nb = gridDim.x, b = blockIdx.x;
+    const int bb = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
+    const int member = bb / blocks_per_member, blk = bb - member * blocks_per_member;
+    const int x0 = (blk % blocks_x) * BL, y0 = (blk / blocks_x) * BL;
+    const float* f = fin + (long long)member * p.member_stride;
+    const int t = threadIdx.x, tx = t % BL_R, ty = t / BL_R;
+    constexpr int PAD = 2 * BL_STEPS;
+    const int i = ((x0 + tx - PAD) % nx + nx) % nx, j = ((y0 + ty - PAD) % ny + ny) % ny;
+    const long long node = (long long)j * nx + i;
+    // exact after s steps: nodes at least `in` from the region's edge
+    const int in = min(min(tx, BL_R - 1 - tx), min(ty, BL_R - 1 - ty));
+    const int lo0 = PAD - 2 * steps;
+    float fc[Q], r = 0.f, u = 0.f, v = 0.f;
+    for (int s = 0; s < steps; ++s) {
+        const int lo = lo0 + 2 * s;
+        float Fx = 0.f, Fy = 0.f;
+        if (in > lo) {
+            if (s == 0) {
+                pull9(f, nodes, wrap(i - 1, nx), i, wrap(i + 1, nx), (long long)wrap(j - 1, ny) * nx,
+                      (long long)j * nx, (long long)wrap(j + 1, ny) * nx, fc);
+            } else {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) fn[q * p.nodes + node] = fc[q];
-    float r, u, v;
-    moments(fc, p.c, r, u, v);
-    ruv[node] = r;
-    ruv[p.nodes + node] = u;
-    ruv[2 * p.nodes + node] = v;
-}
-
-__global__ void k_les(const float* __restrict__ ruv, float* __restrict__ nus, LbmParams p) {
-    const long long node = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (node >= p.nodes) return;
-    const int nx = p.nx, ny = p.ny;
-    const int i = int(node % nx), j = int(node / nx);
-    const float* u = ruv + p.nodes;
-    const float* v = ruv + 2 * p.nodes;
-    const long long e = (long long)j * nx + wrap(i + 1, nx), w = (long long)j * nx + wrap(i - 1, nx);
-    const long long n = (long long)wrap(j + 1, ny) * nx + i, s = (long long)wrap(j - 1, ny) * nx + i;
-    nus[node] = smagorinsky(u[e], u[w], u[n], u[s], v[e], v[w], v[n], v[s], p);
-}
-
-__global__ void k_collide(float* __restrict__ fn, const float* __restrict__ ruv,
-                          const float* __restrict__ nus, const float* __restrict__ force,
-                          LbmParams p) {
-    const long long node = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (node >= p.nodes) return;
-    float fc[Q];
+                for (int q = 0; q < Q; ++q) fc[q] = fs[q][t - (q % 3 - 1) - BL_R * (q / 3 - 1)];
+            }
+            if (FORCE && p.has_force) {
+                Fx = force[(2LL * s) * nodes + node];
+                Fy = force[(2LL * s + 1) * nodes + node];
+            }
+            moments(fc, p.c, r, u, v);
+            su[t] = u;
+            sv[t] = v;
+        }
+        __syncthreads();  // the velocities are in; every pull from fs is done
+        if (in > lo + 1) {
+            const float nut = smagorinsky(su[t + 1], su[t - 1], su[t + BL_R], su[t - BL_R], sv[t + 1], sv[t - 1],
+                                          sv[t + BL_R], sv[t - BL_R], p);
+            collide9<FORCE>(fc, r, u, v, nut, Fx, Fy, p);
+            if (s + 1 < steps) {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) fc[q] = fn[q * p.nodes + node];
-    float Fx = 0.f, Fy = 0.f;
-    if (p.has_force) {
-        Fx = force[node];
-        Fy = force[p.nodes + node];
+                for (int q = 0; q < Q; ++q) fs[q][t] = fc[q];
+            }
+        }
+        if (s + 1 < steps) __syncthreads();
     }
-    collide9<true>(fc, ruv[node], ruv[p.nodes + node], ruv[2 * p.nodes + node], nus[node], Fx, Fy, p);
+    if (in >= PAD && x0 + tx - PAD < nx && y0 + ty - PAD < ny) {
+        float* fo = fout + (long long)member * p.member_stride;
 #pragma unroll
-    for (int q = 0; q < Q; ++q) fn[q * p.nodes + node] = fc[q];
+        for (int q = 0; q < Q; ++q) fo[q * nodes + node] = fc[q];
+    }
 }
 
 // ----------------------------------------------------------------------------
@@ -608,46 +684,108 @@ __global__ void k_collide(float* __restrict__ fn, const float* __restrict__ ruv,
 // members (the reference seeds every member's generator identically,
 // src/data.cu:227-228).  f_x = sum_n amp_n 2 pi ky_n [(r0 kx + r1 ky) sin(th)
 // + (r2 kx + r3 ky) cos(th)], f_y likewise with -kx   (src/data.cu:305-349)
+//
+// The phase is reduced exactly in integers to a multiple of 2 pi / L, L the least
+// common multiple of nx and ny, so its sine and cosine come from a table of L entries
+// (a square grid: nx entries) instead of a reduction and a sincospif per node and mode:
+// 24 steps' draws and fields of a 256^2 grid take 4.6 + 21.6 us, against 19.7 us for each
+// step's with the phases reduced per node (same bits).  Where L is long the table stays in memory, and past
+// FORCE_TABLE_MAX entries the sines are formed in place.
 // ----------------------------------------------------------------------------
-__global__ void k_force_field(const ForceTable* __restrict__ tab, uint64_t seed, float stdev,
-                              const long long* __restrict__ d_step, int step_offset,
-                              float* __restrict__ force, int nx, int ny) {
-    __shared__ float rnd[4][MAX_FORCE_MODES];
-    __shared__ int kxs[MAX_FORCE_MODES], kys[MAX_FORCE_MODES];
-    __shared__ float amps[MAX_FORCE_MODES];
-    const int n = tab->n;
-    const long long step = *d_step + step_offset;
-    for (int m = threadIdx.x; m < n; m += blockDim.x) {
+constexpr long long FORCE_TABLE_MAX = 1 << 20;
+
+// sin and cos of 2 pi k / L
+__device__ __forceinline__ float2 phase_sincos(long long k, long long L) {
+    float2 sc;
+    sincospif(2.f * float(double(k) / double(L)), &sc.x, &sc.y);
+    return sc;
+}
+
+__global__ void k_force_table(float2* __restrict__ table, int L) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < L) table[k] = phase_sincos(k, L);
+}
+
+// a mode's sine and cosine coefficients at the next steps: draws[step][m]; one
+// workgroup per step
+__global__ void k_force_draws(const ForceTable* __restrict__ tab, uint64_t seed, float stdev,
+                              const long long* __restrict__ d_step, int step_offset, float2* __restrict__ draws) {
+    const long long step = *d_step + step_offset + blockIdx.x;
+    for (int m = threadIdx.x; m < tab->n; m += blockDim.x) {
         double z[4];
-        philox_normal4(seed, uint32_t(step), uint32_t(uint64_t(step) >> 32), uint32_t(m),
-                       STREAM_FORCE, z);
-        for (int a = 0; a < 4; ++a) rnd[a][m] = float(z[a] * double(stdev));
-        kxs[m] = int(tab->kx[m]);
-        kys[m] = int(tab->ky[m]);
-        amps[m] = tab->amp[m];
+        float r[4];
+        philox_normal4(seed, uint32_t(step), uint32_t(uint64_t(step) >> 32), uint32_t(m), STREAM_FORCE, z);
+        for (int a = 0; a < 4; ++a) r[a] = float(z[a] * double(stdev));
+        const int kx = int(tab->kx[m]), ky = int(tab->ky[m]);
+        draws[blockIdx.x * MAX_FORCE_MODES + m] = make_float2(r[0] * kx + r[1] * ky, r[2] * kx + r[3] * ky);
     }
-    __syncthreads();
-    const long long node = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long nodes = (long long)nx * ny;
-    if (node >= nodes) return;
-    const int i = int(node % nx), j = int(node / nx);
-    // phase 2 pi (kx x + ky y), x = (i - nx/2)/nx, reduced exactly in integers
-    const long long period = (long long)nx * ny;
+}
+
+// k (a - n/2) mod n
+__device__ __forceinline__ int phase_step(int k, int a, int n) {
+    const long long num = (long long)k * (a - n / 2);
+    const long long r = num >= INT_MIN && num <= INT_MAX ? (long long)(int(num) % n) : num % n;
+    return int(r < 0 ? r + n : r);
+}
+
+// The force fields of consecutive steps, force[step][x, y][node]: a workgroup forms
+// FF_ROWS rows of 256 columns of one step.  TABLE: 2 the table copied to LDS, 1 read
+// from memory, 0 none.
+constexpr int FF_NT = 256, FF_ROWS = 8, FF_LDS = 2048;
+template <int TABLE>
+__global__ __launch_bounds__(FF_NT) void k_force_field(const ForceTable* __restrict__ tab,
+                                                       const float2* __restrict__ draws,
+                                                       const float2* __restrict__ table, long long L,
+                                                       float* __restrict__ force, int nx, int ny) {
+    __shared__ float4 mode[MAX_FORCE_MODES];  // sine and cosine coefficients, x and y amplitudes
+    __shared__ int kxs[MAX_FORCE_MODES];
+    __shared__ int rowk[MAX_FORCE_MODES][FF_ROWS];  // the rows' phases, in units of 1 / ny
+    __shared__ float2 lt[TABLE == 2 ? FF_LDS : 1];
+    const int n = tab->n;
+    const int y0 = blockIdx.y * FF_ROWS;
     const float two_pi = 6.28318530717958647692f;
-    float fx = 0.f, fy = 0.f;
-    for (int m = 0; m < n; ++m) {
-        const int kx = kxs[m], ky = kys[m];
-        long long num = (long long)kx * (i - nx / 2) * ny + (long long)ky * (j - ny / 2) * nx;
-        num %= period;
-        if (num < 0) num += period;
-        float s, c;
-        sincospif(2.f * float(double(num) / double(period)), &s, &c);
-        const float fek = (rnd[0][m] * kx + rnd[1][m] * ky) * s + (rnd[2][m] * kx + rnd[3][m] * ky) * c;
-        fx += amps[m] * two_pi * float(ky) * fek;
-        fy += amps[m] * two_pi * float(-kx) * fek;
+    for (int m = threadIdx.x; m < n; m += FF_NT) {
+        const int kx = int(tab->kx[m]), ky = int(tab->ky[m]);
+        const float2 d = draws[(long long)blockIdx.z * MAX_FORCE_MODES + m];
+        mode[m] = make_float4(d.x, d.y, tab->amp[m] * two_pi * float(ky), tab->amp[m] * two_pi * float(-kx));
+        kxs[m] = kx;
+        for (int r = 0; r < FF_ROWS; ++r) rowk[m][r] = phase_step(ky, y0 + r, ny);
     }
-    force[node] = fx;
-    force[nodes + node] = fy;
+    if (TABLE == 2)
+        for (int k = threadIdx.x; k < L; k += FF_NT) lt[k] = table[k];
+    __syncthreads();
+    const int i = blockIdx.x * FF_NT + threadIdx.x;
+    if (i >= nx) return;
+    const long long lx = L / nx, ly = L / ny;
+    float fx[FF_ROWS] = {}, fy[FF_ROWS] = {};
+    for (int m = 0; m < n; ++m) {
+        const float4 w = mode[m];
+        const long long col = phase_step(kxs[m], i, nx) * lx;
+#pragma unroll
+        for (int r = 0; r < FF_ROWS; ++r) {
+            float2 sc;
+            if (TABLE > 0) {
+                int k = int(col) + rowk[m][r] * int(ly);
+                k = k >= int(L) ? k - int(L) : k;
+                sc = TABLE == 2 ? lt[k] : table[k];
+            } else {
+                const long long k = col + rowk[m][r] * ly;
+                sc = phase_sincos(k >= L ? k - L : k, L);
+            }
+            const float fek = fmaf(w.y, sc.y, w.x * sc.x);
+            fx[r] = fmaf(w.z, fek, fx[r]);
+            fy[r] = fmaf(w.w, fek, fy[r]);
+        }
+    }
+    const long long nodes = (long long)nx * ny;
+    float* out = force + (long long)blockIdx.z * 2 * nodes;
+#pragma unroll
+    for (int r = 0; r < FF_ROWS; ++r) {
+        if (y0 + r >= ny) break;
+        const long long node = (long long)(y0 + r) * nx + i;
+        out[node] = fx[r];
+        out[nodes + node] = fy[r];
+    }
 }
 
 __global__ void k_step_advance(long long* d_step, int n) { *d_step += n; }
@@ -862,11 +1000,44 @@ inline int node_blocks(long long nodes, int nt) { return int((nodes + nt - 1) / 
 
 bool lbm_fused_supported(int nx, int ny) { return nx % TX == 0 && ny % TY == 0; }
 
-hipError_t launch_force_field(Ctx& c, int step_offset) {
-    const int nt = 256;
-    k_force_field<<<node_blocks(c.nodes, nt), nt, 0, c.stream>>>(
-        c.d_force, c.cfg.force_seed, float(c.cfg.force_rand_stdev), c.d_step, step_offset,
-        c.force_xy, c.nx, c.ny);
+int force_batch(int nx, int ny) {
+    // whole multiples of six steps, so that neither two- nor three-step launches are cut;
+    // at least one three-step launch, else no more than 64 MB of fields
+    const long long fit = (64LL << 20) / (8LL * nx * ny);
+    return fit >= 24 ? 24 : (fit >= 6 ? int(fit / 6 * 6) : 3);
+}
+
+static long long force_period(const Ctx& c) { return std::lcm((long long)c.nx, (long long)c.ny); }
+
+long long force_table_entries(const Ctx& c) {
+    const long long L = force_period(c);
+    return c.lp.has_force && L <= FORCE_TABLE_MAX ? L : 0;
+}
+
+hipError_t launch_force_table(Ctx& c) {
+    const int L = int(force_table_entries(c)), nt = 256;
+    if (L == 0) return hipSuccess;
+    k_force_table<<<(L + nt - 1) / nt, nt, 0, c.stream>>>(c.d_force_table, L);
+    return hipGetLastError();
+}
+
+hipError_t launch_force_field(Ctx& c, int step_offset, int steps) {
+    if (steps < 1 || steps > c.force_steps) return hipErrorInvalidValue;
+    k_force_draws<<<steps, 64, 0, c.stream>>>(c.d_force, c.cfg.force_seed, float(c.cfg.force_rand_stdev), c.d_step,
+                                              step_offset, c.d_force_draws);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const long long L = force_period(c);
+    const dim3 grid(unsigned((c.nx + FF_NT - 1) / FF_NT), unsigned((c.ny + FF_ROWS - 1) / FF_ROWS), unsigned(steps));
+#define FORCE_FIELD(T) \
+    k_force_field<T><<<grid, FF_NT, 0, c.stream>>>(c.d_force, c.d_force_draws, c.d_force_table, L, c.force_xy, c.nx, c.ny)
+    if (L > FORCE_TABLE_MAX)
+        FORCE_FIELD(0);
+    else if (L > FF_LDS)
+        FORCE_FIELD(1);
+    else
+        FORCE_FIELD(2);
+#undef FORCE_FIELD
     return hipGetLastError();
 }
 
@@ -880,14 +1051,14 @@ bool lbm_rows_supported(int nx, int ny, int h) {
 }
 
 // one step in full-row strips of h rows
-static hipError_t launch_rows1(Ctx& c, const float* fin, float* fout, int h, bool force) {
+static hipError_t launch_rows1(Ctx& c, const float* fin, float* fout, const float* field, int h, bool force) {
     if (!lbm_rows_supported(c.nx, c.ny, h)) return hipErrorInvalidValue;
     const int strips = c.ny / h;
     const unsigned nb = unsigned(strips * c.M);
     const size_t lds = sizeof(float) * 8 * size_t(c.nx);
 #define LBM_ROWS(HH)                                                                                       \
-    (force ? k_lbm_rows<true, HH><<<nb, c.nx, lds, c.stream>>>(fin, fout, c.force_xy, c.lp, strips)      \
-           : k_lbm_rows<false, HH><<<nb, c.nx, lds, c.stream>>>(fin, fout, c.force_xy, c.lp, strips))
+    (force ? k_lbm_rows<true, HH><<<nb, c.nx, lds, c.stream>>>(fin, fout, field, c.lp, strips)           \
+           : k_lbm_rows<false, HH><<<nb, c.nx, lds, c.stream>>>(fin, fout, field, c.lp, strips))
     switch (h) {
         case 8: LBM_ROWS(8); break;
         case 16: LBM_ROWS(16); break;
@@ -911,88 +1082,134 @@ bool lbm_rows3_supported(int nx, int ny, int h) {
            (long long)nx * ny * Q * 4 < (1LL << 31);
 }
 
-int lbm_launch_steps(const Ctx& c) {
-    const bool force = c.lp.has_force || c.lp.fric_over_dt != 0.f;
-    if (force) return 1;
-    if (c.lbm_tiles_per_block <= -LBM_THREE_STEP) return 3;
-    return c.lbm_tiles_per_block <= -LBM_TWO_STEP ? 2 : 1;
+// The step's shape: `steps` per launch (BL_STEPS: blocks), `rows` of a full-row strip
+// (0: tiles of 64x16, `tiles` per workgroup)
+struct LbmShape {
+    int steps, rows, tiles;
+};
+
+// Time of one strip launch, in arbitrary units: a strip of r rows walks r + halo row
+// iterations, each taking 3 + 2 w with w wavefronts on a SIMD (256^2, three steps: 1.25,
+// 1.85 and 2.75 us at w = 1, 2, 4), in as many generations as the grid needs.
+static double strip_cost(const Ctx& c, int r, int halo, size_t lds_per_column) {
+    const int waves = (c.nx + 63) / 64;
+    const long long wgs = (long long)((c.ny + r - 1) / r) * c.M;
+    const long long per_cu = std::min<long long>((160 * 1024) / (long long)(lds_per_column * c.nx), 16 / waves);
+    const long long slots = 256 * std::max(1LL, per_cu);
+    const double w = std::ceil(double(std::min(wgs, slots)) * waves / 1024.0);
+    return (r + halo) * (3.0 + 2.0 * w) * std::max(1.0, double(wgs) / double(slots));
 }
 
-static hipError_t launch_rows2(Ctx& c, const float* fin, float* fout, int h) {
-    if (!lbm_rows2_supported(c.nx, c.ny, h)) return hipErrorInvalidValue;
-    const int strips = c.ny / h;
-    const unsigned nb = unsigned(strips * c.M);
-    const size_t lds = sizeof(float) * (12 + 3 * P1Q) * size_t(c.nx);
-    const void* fn = h == 16 ? reinterpret_cast<const void*>(&k_lbm_rows2<16>)
-                             : reinterpret_cast<const void*>(&k_lbm_rows2<32>);
+// The shape of a context whose shape was not set.  Measured us per step (256 CUs):
+//                       tiles  blocks  strips (rows)
+//   64^2  x  8           4.7    1.7    4.8 (4)
+//   256^2 x  1           5.2    1.9    5.7 (4)
+//   256^2 x  8           8.2    6.7    7.1 (4)
+//   250x131 x 20        11.2    9.3    8.4 (6)
+//   256^2 x 16          14.2   12.2    9.8 (8)
+//   256^2 x 32          25.9   23.0   13.0 (16)
+//   256^2 x 64          67.4   48.4   24.1 (16)
+//   512^2 x 64           250    193     88 (32)
+//   1024^2 x 4          69.3   49.3   34.2 (16, two steps)
+//   2048x1024 x 1       26.4   23.1     -
+// So: blocks up to about nine per CU (a block steps nearly twice its own nodes, which
+// costs nothing while the chip is not full) and for rows longer than a workgroup;
+// strips elsewhere, their height by strip_cost.
+static LbmShape default_shape(const Ctx& c) {
+    const LbmShape blocks{BL_STEPS, 0, 1};
+    const long long nb = (long long)((c.nx + BL - 1) / BL) * ((c.ny + BL - 1) / BL) * c.M;
+    const bool small = c.nx < 8 || c.ny < 16;  // a strip's halo wraps around at most once
+    if (c.nx > 1024 || small || nb <= 9 * 256 || (long long)c.nx * c.ny * Q * 4 >= (1LL << 31)) return blocks;
+    const bool three = c.nx <= 512;
+    LbmShape best = blocks;
+    double cost = 0;
+    for (int r : {4, 6, 8, 12, 16, 24, 32}) {
+        const double t = three ? strip_cost(c, r, 10, 36 * 4) : strip_cost(c, r, 6, (12 + 3 * P1Q) * 4);
+        if (best.rows == 0 || t < cost) {
+            best = {three ? 3 : 2, r, 0};
+            cost = t;
+        }
+    }
+    return best;
+}
+
+static LbmShape lbm_shape(const Ctx& c) {
+    const int code = c.lbm_tiles_per_block;
+    if (code <= -LBM_THREE_STEP) return {3, -code - LBM_THREE_STEP, 0};
+    if (code <= -LBM_TWO_STEP) return {2, -code - LBM_TWO_STEP, 0};
+    if (code < 0) return {1, -code, 0};
+    return code > 1 ? LbmShape{1, 0, code} : default_shape(c);
+}
+
+int lbm_launch_steps(const Ctx& c) { return lbm_shape(c).steps; }
+
+template <class K>
+static hipError_t launch_strips(K kernel, Ctx& c, const float* fin, float* fout, const float* force, int rows,
+                                size_t lds_per_column) {
+    const int strips = (c.ny + rows - 1) / rows;
+    const size_t lds = lds_per_column * size_t(c.nx);
     if (lds > 65536) {  // beyond the default dynamic LDS of a workgroup
-        const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
     }
-    if (h == 16)
-        k_lbm_rows2<16><<<nb, c.nx, lds, c.stream>>>(fin, fout, c.lp, strips);
-    else
-        k_lbm_rows2<32><<<nb, c.nx, lds, c.stream>>>(fin, fout, c.lp, strips);
+    kernel<<<unsigned(strips * c.M), unsigned((c.nx + 63) / 64 * 64), lds, c.stream>>>(fin, fout, force, c.lp, strips,
+                                                                                       rows);
     return hipGetLastError();
 }
 
-static hipError_t launch_rows3(Ctx& c, const float* fin, float* fout, int h) {
-    if (!lbm_rows3_supported(c.nx, c.ny, h)) return hipErrorInvalidValue;
-    const int strips = c.ny / h;
-    const unsigned nb = unsigned(strips * c.M);
-    const size_t lds = sizeof(float) * 36 * size_t(c.nx);
-    const bool n256 = c.nx == 256;
-    const void* fn = h == 16 ? (n256 ? reinterpret_cast<const void*>(&k_lbm_rows3<16, 256>)
-                                     : reinterpret_cast<const void*>(&k_lbm_rows3<16, 0>))
-                             : (n256 ? reinterpret_cast<const void*>(&k_lbm_rows3<32, 256>)
-                                     : reinterpret_cast<const void*>(&k_lbm_rows3<32, 0>));
-    if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-        if (e != hipSuccess) return e;
+static hipError_t launch_rows2(Ctx& c, const float* fin, float* fout, const float* force, int rows) {
+    const bool fr = c.lp.has_force || c.lp.fric_over_dt != 0.f;
+    const size_t lds = sizeof(float) * (12 + 3 * P1Q);
+    if (!fr && lbm_rows2_supported(c.nx, c.ny, rows))
+        return rows == 16 ? launch_strips(&k_lbm_rows2<16, false>, c, fin, fout, force, rows, lds)
+                          : launch_strips(&k_lbm_rows2<32, false>, c, fin, fout, force, rows, lds);
+    return fr ? launch_strips(&k_lbm_rows2<0, true>, c, fin, fout, force, rows, lds)
+              : launch_strips(&k_lbm_rows2<0, false>, c, fin, fout, force, rows, lds);
+}
+
+static hipError_t launch_rows3(Ctx& c, const float* fin, float* fout, const float* force, int rows) {
+    const bool fr = c.lp.has_force || c.lp.fric_over_dt != 0.f;
+    const size_t lds = sizeof(float) * 36;
+    if (!fr && lbm_rows3_supported(c.nx, c.ny, rows)) {
+        if (c.nx == 256)
+            return rows == 16 ? launch_strips(&k_lbm_rows3<16, 256, false>, c, fin, fout, force, rows, lds)
+                              : launch_strips(&k_lbm_rows3<32, 256, false>, c, fin, fout, force, rows, lds);
+        return rows == 16 ? launch_strips(&k_lbm_rows3<16, 0, false>, c, fin, fout, force, rows, lds)
+                          : launch_strips(&k_lbm_rows3<32, 0, false>, c, fin, fout, force, rows, lds);
     }
-    if (h == 16 && n256)
-        k_lbm_rows3<16, 256><<<nb, c.nx, lds, c.stream>>>(fin, fout, c.lp, strips);
-    else if (h == 16)
-        k_lbm_rows3<16, 0><<<nb, c.nx, lds, c.stream>>>(fin, fout, c.lp, strips);
-    else if (n256)
-        k_lbm_rows3<32, 256><<<nb, c.nx, lds, c.stream>>>(fin, fout, c.lp, strips);
+    return fr ? launch_strips(&k_lbm_rows3<0, 0, true>, c, fin, fout, force, rows, lds)
+              : launch_strips(&k_lbm_rows3<0, 0, false>, c, fin, fout, force, rows, lds);
+}
+
+static hipError_t launch_blocks(Ctx& c, const float* fin, float* fout, const float* force, int steps) {
+    const int bx = (c.nx + BL - 1) / BL, blocks = bx * ((c.ny + BL - 1) / BL);
+    if (c.lp.has_force || c.lp.fric_over_dt != 0.f)
+        k_lbm_block<true><<<unsigned(blocks * c.M), BL_R * BL_R, 0, c.stream>>>(fin, fout, force, c.lp, bx, blocks, steps);
     else
-        k_lbm_rows3<32, 0><<<nb, c.nx, lds, c.stream>>>(fin, fout, c.lp, strips);
+        k_lbm_block<false><<<unsigned(blocks * c.M), BL_R * BL_R, 0, c.stream>>>(fin, fout, force, c.lp, bx, blocks, steps);
     return hipGetLastError();
 }
 
-hipError_t launch_lbm_fused(Ctx& c, const float* fin, float* fout, int steps) {
-    const bool force = c.lp.has_force || c.lp.fric_over_dt != 0.f;
-    if (steps < 1 || steps > lbm_launch_steps(c)) return hipErrorInvalidValue;
-    if (c.lbm_tiles_per_block <= -LBM_TWO_STEP) {
-        // full-row strips of h rows taking three (or two) steps per launch, or one,
-        // for the last steps of a forecast or a forced flow
-        const int h = -c.lbm_tiles_per_block - (c.lbm_tiles_per_block <= -LBM_THREE_STEP ? LBM_THREE_STEP : LBM_TWO_STEP);
-        if (steps == 3) return launch_rows3(c, fin, fout, h);
-        if (steps == 2) return launch_rows2(c, fin, fout, h);
-        return launch_rows1(c, fin, fout, h, force);
-    }
-    if (c.lbm_tiles_per_block < 0) return launch_rows1(c, fin, fout, -c.lbm_tiles_per_block, force);
-    const int tiles_x = c.nx / TX, tiles_y = c.ny / TY;
-    const int tiles = tiles_x * tiles_y;
-    const int total = tiles * c.M;
-    const int per_block = c.lbm_tiles_per_block;
-    if (per_block < 1 || total % per_block != 0) return hipErrorInvalidValue;
-    const int nb = total / per_block;
-    if (force)
-        k_lbm_fused<true><<<nb, NT, 0, c.stream>>>(fin, fout, c.force_xy, c.lp, tiles_x, tiles, per_block);
+hipError_t launch_lbm_fused(Ctx& c, const float* fin, float* fout, int steps, const float* force) {
+    const LbmShape sh = lbm_shape(c);
+    if (steps < 1 || steps > sh.steps) return hipErrorInvalidValue;
+    if (sh.steps == BL_STEPS) return launch_blocks(c, fin, fout, force, steps);
+    if (steps == 3) return launch_rows3(c, fin, fout, force, sh.rows);
+    if (steps == 2) return launch_rows2(c, fin, fout, force, sh.rows);
+    const bool fr = c.lp.has_force || c.lp.fric_over_dt != 0.f;
+    if (sh.rows > 0 && lbm_rows_supported(c.nx, c.ny, sh.rows)) return launch_rows1(c, fin, fout, force, sh.rows, fr);
+    const bool ragged = !lbm_fused_supported(c.nx, c.ny);
+    const int tiles_x = (c.nx + TX - 1) / TX, tiles = tiles_x * ((c.ny + TY - 1) / TY);
+    const int total = tiles * c.M, per_block = ragged || sh.tiles < 1 ? 1 : sh.tiles;
+    if (total % per_block != 0) return hipErrorInvalidValue;
+#define LBM_TILES(FF, RR) \
+    k_lbm_fused<FF, RR><<<total / per_block, NT, 0, c.stream>>>(fin, fout, force, c.lp, tiles_x, tiles, per_block)
+    if (ragged)
+        fr ? LBM_TILES(true, true) : LBM_TILES(false, true);
     else
-        k_lbm_fused<false><<<nb, NT, 0, c.stream>>>(fin, fout, c.force_xy, c.lp, tiles_x, tiles, per_block);
-    return hipGetLastError();
-}
-
-hipError_t launch_lbm_plain_member(Ctx& c, const float* fin, float* fout, int member) {
-    const int nt = 256;
-    const int nb = node_blocks(c.nodes, nt);
-    const long long off = (long long)member * c.lp.member_stride;
-    k_stream_macro<<<nb, nt, 0, c.stream>>>(fin + off, fout + off, c.plain_ruv, c.lp);
-    k_les<<<nb, nt, 0, c.stream>>>(c.plain_ruv, c.plain_nus, c.lp);
-    k_collide<<<nb, nt, 0, c.stream>>>(fout + off, c.plain_ruv, c.plain_nus, c.force_xy, c.lp);
+        fr ? LBM_TILES(true, false) : LBM_TILES(false, false);
+#undef LBM_TILES
     return hipGetLastError();
 }
 

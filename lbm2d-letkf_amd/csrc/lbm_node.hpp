@@ -100,19 +100,24 @@ __device__ __forceinline__ void collide9(float fc[Q], float rho, float u, float 
     LBMNODE_CONTRACT_PER_STATEMENT
     const float tau = 0.5f + p.k_tau * (p.nu + nut);
     const float omega = __builtin_amdgcn_rcpf(tau);  // 1 ulp
-    const float fxp = (Fx - p.fric_over_dt * u) * p.dt;
-    const float fyp = (Fy - p.fric_over_dt * v) * p.dt;
     float feq[Q];
     equilibrium9(rho, u, v, p, feq);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int ex = q % 3 - 1, ey = q / 3 - 1;
-        const float wq = (ex == 0 && ey == 0) ? W0 : ((ex == 0 || ey == 0) ? W1 : W2);
-        const float fq = fc[q] - omega * (fc[q] - feq[q]);
-        if constexpr (FORCE)
-            fc[q] = fq + wq * rho * p.force_scale * (float(ex) * fxp + float(ey) * fyp);
-        else
-            fc[q] = fq;
+    for (int q = 0; q < Q; ++q) fc[q] = fc[q] - omega * (fc[q] - feq[q]);
+    if constexpr (FORCE) {
+        // w_q rho force_scale (e_x fx + e_y fy): opposite directions share it up to the sign
+        const float fxp = (Fx - p.fric_over_dt * u) * p.dt;
+        const float fyp = (Fy - p.fric_over_dt * v) * p.dt;
+        const float a1 = W1 * rho * p.force_scale, a2 = W2 * rho * p.force_scale;
+        const float fp = fxp + fyp, fm = fxp - fyp;
+        fc[5] = fc[5] + a1 * fxp;
+        fc[3] = fc[3] - a1 * fxp;
+        fc[7] = fc[7] + a1 * fyp;
+        fc[1] = fc[1] - a1 * fyp;
+        fc[8] = fc[8] + a2 * fp;
+        fc[0] = fc[0] - a2 * fp;
+        fc[2] = fc[2] + a2 * fm;
+        fc[6] = fc[6] - a2 * fm;
     }
 }
 
