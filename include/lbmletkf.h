@@ -100,7 +100,8 @@ typedef struct lbmletkf_config {
     double closure_strain_scale; /* MLP inputs are strain components / this scale            */
     double closure_nu_scale;     /* MLP output nu_t = this scale * softplus(z)               */
     double closure_nu_max;       /* nu_t above this (or not finite) falls back to Smagorinsky */
-    /* MIXED: FP32 stop tolerance (0: 3e-6).  Without FP64 sweeps the phase stops
+    /* MIXED, where the sweeps are taken (FP64 sweeps requested, a dumped gridpoint, or a
+     * local problem of condition above 1023): FP32 stop tolerance (0: 3e-6).  Without FP64 sweeps the phase stops
      * once the columns' largest pair cosine, measured after a sweep, is at most a
      * third of this, or one sweep after that measurement, below 1e-4, stops halving;
      * with FP64 sweeps it stops after the sweep whose largest pair cosine met is at
@@ -255,13 +256,14 @@ int lbmletkf_get_obs_ensemble(lbmletkf_ctx* ctx, float* dy, float* dyo);
  * src/main.cu:95-115, src/letkf.cu:120-360).  enable(1) clears and starts them.
  * Phases: "forecast" (all LBM kernels incl. forcing), "obs" (H(x), innovations),
  * "gram" (PLAIN: C and b), "solve" (PLAIN: eigensolve, transform, state update;
- * MIXED: gather, MFMA Gram and the FP32 Jacobi sweeps), "finish" (MIXED: FP64
- * sweeps, transform, state update).
+ * MIXED: gather, MFMA Gram and the update by series, or the FP32 Jacobi sweeps),
+ * "finish" (MIXED: FP64 sweeps, transform, state update).
  * read() returns the accumulated seconds, the number of kernel launches and a
  * work count: node updates (forecast), observations (obs), local scalar
  * observations summed over gridpoints (gram), Jacobi sweeps summed over
- * gridpoints (solve; FP32 sweeps in MIXED).  The pseudo-phase "solve_fp64" reads
- * the MIXED variant's FP64 sweeps summed over gridpoints as its work count.
+ * gridpoints (solve; FP32 sweeps in MIXED, where the series leaves any).  The
+ * pseudo-phases "solve_fp64" and "solve_series" read the MIXED variant's FP64 sweeps
+ * and the block products of its series, summed over gridpoints, as their work count.
  * read() synchronises the stream.  While timing is on, lbmletkf_cycle launches
  * eagerly instead of replaying its graph. */
 int lbmletkf_profile_enable(lbmletkf_ctx* ctx, int on);

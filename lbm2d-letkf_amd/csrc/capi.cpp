@@ -363,6 +363,11 @@ int ensure_mixed_buffers(Ctx* c) {
         HIP_TRY(c, dalloc(&c->d_mix_u, (size_t)c->nodes * N * N));
         HIP_TRY(c, dalloc(&c->d_mix_b, (size_t)c->nodes * N));
     }
+    if (mixed_fused(*c) && !c->d_series) {
+        HIP_TRY(c, hipMalloc(&c->d_series, series_table_bytes()));
+        HIP_TRY(c, hipMemcpy(c->d_series, series_table_host(), series_table_bytes(), hipMemcpyHostToDevice));
+        HIP_TRY(c, dalloc(&c->d_left, c->nodes));
+    }
     c->mix_width = N;
     return LBMLETKF_OK;
 }
@@ -485,7 +490,7 @@ int analysis_launches(Ctx* c) {
         hipEvent_t e2 = prof_begin(c);
         HIP_TRY(c, launch_letkf_mixed(*c, c->f[c->cur], c->prof ? c->d_sweeps : nullptr, nullptr,
                                       c->cfg.gram_passes, nullptr, nullptr));
-        prof_end(c, PH_SOLVE, e2, 1, 0);
+        prof_end(c, PH_SOLVE, e2, 2, 0);
         c->dump_kind = 1;
         return LBMLETKF_OK;
     }
@@ -572,7 +577,7 @@ Ctx::~Ctx() {
     void* ptrs[] = {f[0], f[1], force_xy, d_force_draws, d_force_table, d_force, d_step, d_status,
                     d_site_node, d_loc_ptr, d_loc_site, d_loc_w, d_obs_coef, d_yo, d_hx, d_hx1, d_dy,
                     d_dyo, d_gram, d_bvec, d_mix_u, d_mix_b, d_dump, d_red, d_truth, d_sweeps,
-                    d_sweeps64, d_closure, d_site_map, d_ens_uv, d_ens_out};
+                    d_sweeps64, d_series_steps, d_closure, d_series, d_left, d_site_map, d_ens_uv, d_ens_out};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (const ProfRec& r : prof_pending) {
@@ -1255,6 +1260,8 @@ int lbmletkf_profile_enable(lbmletkf_ctx* ctx, int on) {
     }
     if (!c->d_sweeps) HIP_TRY(c, dalloc(&c->d_sweeps, 1));
     if (!c->d_sweeps64) HIP_TRY(c, dalloc(&c->d_sweeps64, 1));
+    if (!c->d_series_steps) HIP_TRY(c, dalloc(&c->d_series_steps, 1));
+    HIP_TRY(c, hipMemset(c->d_series_steps, 0, sizeof(unsigned long long)));
     HIP_TRY(c, hipMemset(c->d_sweeps, 0, sizeof(unsigned long long)));
     HIP_TRY(c, hipMemset(c->d_sweeps64, 0, sizeof(unsigned long long)));
     c->prof = on != 0;
@@ -1272,10 +1279,13 @@ int lbmletkf_profile_read(lbmletkf_ctx* ctx, const char* phase, double* seconds,
         if (std::strcmp(phase, names[p]) == 0) ph = p;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     if (int st = prof_collect(c)) return st;
-    if (std::strcmp(phase, "solve_fp64") == 0) {
-        // FP64 sweeps of the MIXED variant (its time is part of "solve")
+    const bool series = std::strcmp(phase, "solve_series") == 0;
+    if (series || std::strcmp(phase, "solve_fp64") == 0) {
+        // block products of the series, or FP64 sweeps, of the MIXED variant (their time is
+        // part of "solve")
         unsigned long long sw = 0;
-        if (c->d_sweeps64) HIP_TRY(c, hipMemcpy(&sw, c->d_sweeps64, sizeof(sw), hipMemcpyDeviceToHost));
+        const unsigned long long* d = series ? c->d_series_steps : c->d_sweeps64;
+        if (d) HIP_TRY(c, hipMemcpy(&sw, d, sizeof(sw), hipMemcpyDeviceToHost));
         if (seconds) *seconds = 0.0;
         if (launches) *launches = 0;
         if (work) *work = (long long)sw;

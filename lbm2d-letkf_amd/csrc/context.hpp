@@ -119,6 +119,8 @@ struct Ctx {
     float* d_mix_u = nullptr;     // [nodes][N][N] FP32 columns of U = C V after the FP32 sweeps
     float* d_mix_b = nullptr;     // [nodes][N] b = dY^T R^-1 dyo
     int mix_width = 0;
+    float4* d_series = nullptr;   // coefficients of the fused form's series (letkf_series.hpp)
+    unsigned char* d_left = nullptr;  // [nodes] gridpoints the series left to the sweeps
     int mix_chain = 8;            // consecutive gridpoints per wavefront in k_mixed_solve
     // shape of the LBM step: 1 the rule of lbm.hip on the grid and ensemble size (blocks
     // or strips), k > 1 tiles of 64x16 per workgroup (k_lbm_fused),
@@ -156,6 +158,7 @@ struct Ctx {
     long long prof_work[PH_COUNT] = {};
     unsigned long long* d_sweeps = nullptr;    // Jacobi sweeps summed over gridpoints
     unsigned long long* d_sweeps64 = nullptr;  // MIXED: FP64 sweeps summed over gridpoints
+    unsigned long long* d_series_steps = nullptr;  // MIXED: block products of the series summed over gridpoints
     int dump_kind = 0;  // 0: W, w, evals (plain); 1: V, d, b (mixed), assembled on the host
 
     // MIXED cycle (analysis + da_interval steps) as an instantiated hipGraph, one per
@@ -234,6 +237,9 @@ hipError_t launch_solve_fp64(Ctx& c, float* f, unsigned long long* sweeps);
 
 // ---- launchers (letkf_mixed.hip) ----------------------------------------------
 int mixed_width(int M);
+// the coefficient table of the fused form's series, for Ctx::d_series
+size_t series_table_bytes();
+const float* series_table_host();
 // the presets' form: one fused kernel (no FP64 sweeps requested)
 bool mixed_fused(const Ctx& c);
 long long mixed_fused_blocks(int nx, int ny, int chain);

@@ -1002,8 +1002,9 @@ bool lbm_fused_supported(int nx, int ny) { return nx % TX == 0 && ny % TY == 0; 
 
 int force_batch(int nx, int ny) {
     // whole multiples of six steps, so that neither two- nor three-step launches are cut;
-    // at least one three-step launch, else no more than 64 MB of fields
-    const long long fit = (64LL << 20) / (8LL * nx * ny);
+    // at least one three-step launch, else no more than 16 MB of fields (they are read back
+    // from L2, and allocating more takes longer than the launches it saves)
+    const long long fit = (16LL << 20) / (8LL * nx * ny);
     return fit >= 24 ? 24 : (fit >= 6 ? int(fit / 6 * 6) : 3);
 }
 

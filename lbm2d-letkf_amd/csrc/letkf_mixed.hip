@@ -1,6 +1,16 @@
 // Mixed-precision LETKF analysis for gfx950: the local analysis of
-// src/util/letkf_solver.h:235-349 at every gridpoint, one wavefront per gridpoint,
-// in two kernels:
+// src/util/letkf_solver.h:235-349 at every gridpoint, one wavefront per gridpoint.
+//
+// Without FP64 sweeps (the presets):
+// k_series_analysis: gather, Gram matrix on the matrix cores, and the update by
+//     Chebyshev series of C (letkf_series.hpp), matrix products throughout; then
+// k_mixed_analysis: gather, Gram matrix, FP32 Jacobi sweeps and update of the
+//     gridpoints the series left (condition number above 1023, or dumped: the dump
+//     records eigenpairs).
+// At 256^2 x 64 (kappa ~ 20) the first takes 1.2 ms and the second, with nothing left
+// to do, 9 us; the sweeps take 5.1 ms for the same gridpoints.
+//
+// With FP64 sweeps, two kernels:
 //
 // k_mixed_solve (FP32, ~200 VGPRs, C in 16 KB of LDS; a chain of neighbouring
 // gridpoints per wavefront, each warm-started from its predecessor's eigenvectors)
@@ -31,16 +41,14 @@
 //
 // The workspace round trip (4 N^2 bytes per gridpoint each way) costs ~0.3 ms at
 // 256^2 x 64 and lets each kernel have the register budget of its own phase.
+#include <cstring>
+
 #include "context.hpp"
+#include "letkf_series.hpp"
 
 namespace lbmletkf {
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 struct MixedParams {
     int M, nodes, n_vars;
@@ -58,6 +66,9 @@ struct MixedParams {
     int dump_g0, dump_n;
     int chain;              // k_mixed_solve: consecutive gridpoints per wavefront
     int write_state;        // k_mixed_analysis: 0 skips the state update (timing only)
+    const float4* series;   // k_series_analysis: coefficients of the series (letkf_series.hpp)
+    float series_scale;     // the power of two that brings diag to [1, 2)
+    unsigned long long* series_steps;  // block products summed over gridpoints (may be null)
     unsigned long long* sweeps32;
     unsigned long long* sweeps64;
 };
@@ -74,10 +85,11 @@ struct MixedTask {
     float* f;
     double* dump;
     int* status;
+    unsigned char* left;
     MixedParams mp;
     int N;
-    int b0_solve, nb_solve;    // workgroup range of k_mixed_solve_group
-    int b0_finish, nb_finish;  // workgroup range of k_mixed_finish_group
+    int b0_solve, nb_solve;    // workgroup range of k_mixed_solve_group and k_mixed_analysis_group
+    int b0_finish, nb_finish;  // workgroup range of k_mixed_finish_group and k_series_analysis_group
 };
 struct MixedGroup {
     int n;
@@ -576,7 +588,7 @@ __device__ __forceinline__ void gram_acc(int g, int lane, const int* __restrict_
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(dy), 0, mp.n_obs * M * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t rdyo =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(dyo), 0, mp.n_obs * 4, 0x00020000);
-    const float cmask = col == 0 ? 1.f : 0.f;
+    const float cmask = col == 9 ? 1.f : 0.f;  // b in column 9 of its tiles
     for (int base = 0; base < P; base += 32) {
         const int jj0 = base + 8 * kq;
         int e = e0 + jj0 / nv, va = jj0 % nv;
@@ -707,7 +719,7 @@ __device__ inline void gram_to_lds(int g, int lane, const int* __restrict__ loc_
     }
 #pragma unroll
     for (int I = 0; I < NT; ++I)
-        if (col == 0) {
+        if (col == 9) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) bg[16 * I + 4 * kq + r] = acc[NTILE + I][r];
         }
@@ -908,7 +920,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 }
 
 // ---------------------------------------------------------------------------------
-// The fused analysis (the presets: no FP64 sweeps).  The gather, Gram and FP32
+// The fused analysis by sweeps (no FP64 sweeps).  The gather, Gram and FP32
 // sweeps of k_mixed_solve, then in the same wavefront the eigenpairs and the update
 // of the gridpoint's members:
 //   lambda_i = ||u_i||, v_i = u_i / lambda_i          (column norms in FP64)
@@ -1099,13 +1111,115 @@ __device__ inline void warm_start_acc(const f32x4 (&acc)[GRAM_FULL<N>], float* c
             for (int r = 0; r < 4; ++r) cv[(16 * ti + 4 * kq + r) * N + 16 * tj + col] = d[ti * NT + tj][r];
 }
 
+// ---------------------------------------------------------------------------------
+// The analysis by series (letkf_series.hpp), one wavefront per gridpoint, nothing
+// carried from one gridpoint to the next: gather and Gram matrix as above, then lane
+// (c, grp) takes variable c of members 16 T + 4 grp + r (c < 9), column 9 of the block
+// is b.  left[g] tells the kernel of the sweeps what it still has to do: the gridpoints
+// whose local problem is too badly conditioned for the series, and those dumped.
+// ---------------------------------------------------------------------------------
+template <int N>
+struct SeriesShared {
+    float basis[N == 64 ? 4 * 64 * 16 : 4];
+};
+
+template <int N, int PASSES>
+__device__ __forceinline__ void series_body(int bx, int nbx, const int* __restrict__ loc_ptr,
+                                            const int* __restrict__ loc_site, const float* __restrict__ loc_w,
+                                            const float* __restrict__ dy, const float* __restrict__ dyo,
+                                            float* __restrict__ f, const MixedParams& mp, int* __restrict__ status,
+                                            unsigned char* __restrict__ left, float* lds) {
+    constexpr int NT = N / 16;
+    const int lane = threadIdx.x;
+    const int g = xcd_order(bx, nbx);
+    if (g >= mp.nodes) return;
+    const int M = mp.M;
+    const bool dumped = mp.write_state && g >= mp.dump_g0 && g < mp.dump_g0 + mp.dump_n;
+    if (dumped) {
+        if (lane == 0) left[g] = 1;
+        return;
+    }
+    f32x4 acc[GRAM_FULL<N>];
+    gram_acc<N, PASSES, true>(g, lane, loc_ptr, loc_site, loc_w, dy, dyo, mp, acc);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // addresses formed here, not held through the Gram matrix
+    const int c = ln & 15, grp = ln >> 4;
+    const float* fq = f + (long long)(c < Q ? c : 0) * mp.nodes + g;
+    f32x4 r[NT];
+    double sum = 0.0;
+#pragma unroll
+    for (int T = 0; T < NT; ++T)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int l = 16 * T + 4 * grp + k;
+            r[T][k] = fq[(long long)(l < M ? l : 0) * mp.member_stride];
+            sum += l < M ? double(r[T][k]) : 0.0;
+        }
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    const double xbar = sum / double(M);
+#pragma unroll
+    for (int T = 0; T < NT; ++T)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bool in = 16 * T + 4 * grp + k < M;
+            const float dx = c < Q && in ? float(double(r[T][k]) - xbar) : 0.f;
+            r[T][k] = c == 9 ? acc[NT * NT + T][k] : dx;
+        }
+    SeriesBasis<N> basis(lds, lane);
+    const int steps = series_apply<N>(acc, r, mp.diag, mp.series_scale, mp.series, basis, lane);
+    if (lane == 0) {
+        left[g] = steps == 0;
+        if (mp.series_steps) atomicAdd(mp.series_steps, (unsigned long long)steps);
+    }
+    if (steps == 0) return;
+    // dX w = sum_k dX[k] w[k], w = C^-1 b in column 9 (row_newbcast:9)
+    float dw = 0.f;
+#pragma unroll
+    for (int T = 0; T < NT; ++T) {
+        const f32x4 dx = basis.get(0, T);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            dw = fmaf(dx[k], __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(r[T][k]), 0x159, 0xF, 0xF, true)),
+                      dw);
+    }
+    dw += __shfl_xor(dw, 16);
+    dw += __shfl_xor(dw, 32);
+    asm volatile("" : "+v"(ln));  // the addresses again, for the same reason
+    const int co = ln & 15, go = ln >> 4;
+    if (mp.write_state && co < Q) {
+        const float s = float(mp.sqm1);
+        float* fo = f + (long long)co * mp.nodes + g + 4 * go * mp.member_stride;
+        bool bad = false;
+#pragma unroll
+        for (int T = 0; T < NT; ++T)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (16 * T + 4 * go + k >= M) continue;
+                const float xa = float(xbar + double(fmaf(s, r[T][k], dw)));
+                bad |= !isfinite(xa);
+                fo[(16 * T + k) * mp.member_stride] = xa;
+            }
+        if (bad) atomicOr(status, 1);
+    }
+}
+
+template <int N, int PASSES>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_series_analysis(
+    const int* __restrict__ loc_ptr, const int* __restrict__ loc_site, const float* __restrict__ loc_w,
+    const float* __restrict__ dy, const float* __restrict__ dyo, float* __restrict__ f, MixedParams mp,
+    int* __restrict__ status, unsigned char* __restrict__ left) {
+    __shared__ __align__(16) SeriesShared<N> sh;
+    series_body<N, PASSES>(blockIdx.x, gridDim.x, loc_ptr, loc_site, loc_w, dy, dyo, f, mp, status, left, sh.basis);
+}
+
 template <int N, int PASSES>
 __device__ __forceinline__ void analysis_body(int bx, int nbx, const int* __restrict__ loc_ptr,
                                               const int* __restrict__ loc_site, const float* __restrict__ loc_w,
                                               const float* __restrict__ dy, const float* __restrict__ dyo,
                                               float* __restrict__ f, const MixedParams& mp,
                                               double* __restrict__ dump, int* __restrict__ status,
-                                              FusedShared<N>& sh) {
+                                              const unsigned char* __restrict__ left, FusedShared<N>& sh) {
     constexpr int NT = N / 16;
     const int lane = threadIdx.x;
     const int M = mp.M;
@@ -1119,22 +1233,27 @@ __device__ __forceinline__ void analysis_body(int bx, int nbx, const int* __rest
     const int gy1 = min(gy0 + mp.chain, mp.ny);
     bool bad = false;
     int sweeps = 2;
+    bool warm = false;  // the previous gridpoint of the chain left its eigenvectors in cv
     for (int gy = gy0; gy < gy1; ++gy) {
         const int g = gy * mp.nx + gx;
+        if (!left[g]) {
+            warm = false;
+            continue;
+        }
         f32x4 acc[GRAM_FULL<N>];
         gram_acc<N, PASSES, true>(g, lane, loc_ptr, loc_site, loc_w, dy, dyo, mp, acc);
         gram_add_diag<N>(acc, lane, M, mp.diag);
         if (mp.write_state && g >= mp.dump_g0 && g < mp.dump_g0 + mp.dump_n)
             dump_c_acc<N>(acc, dump + (long long)(g - mp.dump_g0) * dump_record(M) + M * M + 2 * M, M, lane);
         __syncthreads();  // the previous gridpoint's reads of stage and coef are done
-        if ((lane & 15) == 0) {
+        if ((lane & 15) == 9) {
 #pragma unroll
             for (int I = 0; I < NT; ++I)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) sh.bvec[16 * I + 4 * (lane >> 4) + r] = acc[NT * NT + I][r];
         }
-        // U0: C itself for the first gridpoint of the chain, else C V_prev
-        if (gy == gy0)
+        // U0: C itself, or after a gridpoint that left its eigenvectors C V_prev
+        if (!warm)
             gram_to_cv<N>(acc, sh.cv, lane);
         else
             warm_start_acc<N>(acc, sh.cv, lane);
@@ -1146,8 +1265,9 @@ __device__ __forceinline__ void analysis_body(int bx, int nbx, const int* __rest
         // fall ~0.1 -> 1e-3 -> floor, and a measurement that fails costs about a
         // seventh of a sweep (0.22 ms per analysis at 256^2 x 64 when made after
         // every warm start's second sweep).
-        const int first = gy == gy0 ? 2 : min(max(sweeps, 2), 3);
+        const int first = !warm ? 2 : min(max(sweeps, 2), 3);
         const float uscale = jacobi_fp32<N, true>(u, sc, sh.cv, lane, mp, sh.cv, first, sweeps);
+        warm = true;
 
         // ---- eigenpairs: lambda_i = ||u_i|| in FP64, v_i = u_i / ||u_i|| ------------------
         double n4[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1286,9 +1406,9 @@ template <int N, int PASSES>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_mixed_analysis(
     const int* __restrict__ loc_ptr, const int* __restrict__ loc_site, const float* __restrict__ loc_w,
     const float* __restrict__ dy, const float* __restrict__ dyo, float* __restrict__ f, MixedParams mp,
-    double* __restrict__ dump, int* __restrict__ status) {
+    double* __restrict__ dump, int* __restrict__ status, const unsigned char* __restrict__ left) {
     __shared__ __align__(16) FusedShared<N> sh;
-    analysis_body<N, PASSES>(blockIdx.x, gridDim.x, loc_ptr, loc_site, loc_w, dy, dyo, f, mp, dump, status, sh);
+    analysis_body<N, PASSES>(blockIdx.x, gridDim.x, loc_ptr, loc_site, loc_w, dy, dyo, f, mp, dump, status, left, sh);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1571,6 +1691,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 }
 
 template <int PASSES>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_series_analysis_group(MixedGroup G) {
+    int k = 0;
+    while (k + 1 < G.n && int(blockIdx.x) >= G.t[k + 1].b0_finish) ++k;
+    const MixedTask& T = G.t[k];
+    const int bx = int(blockIdx.x) - T.b0_finish;
+    __shared__ __align__(16) SeriesShared<64> sh;
+    switch (T.N) {
+        case 16: series_body<16, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status, T.left, sh.basis); break;
+        case 32: series_body<32, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status, T.left, sh.basis); break;
+        default: series_body<64, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status, T.left, sh.basis); break;
+    }
+}
+
+template <int PASSES>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_mixed_analysis_group(MixedGroup G) {
     int k = 0;
     while (k + 1 < G.n && int(blockIdx.x) >= G.t[k + 1].b0_solve) ++k;
@@ -1586,16 +1720,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     float* tf = T.f;
     double* td = T.dump;
     int* ts = T.status;
+    const unsigned char* tl = T.left;
     switch (T.N) {
         case 16:
-            analysis_body<16, PASSES>(bx, T.nb_solve, lp, ls, lw, ty, to, tf, T.mp, td, ts,
+            analysis_body<16, PASSES>(bx, T.nb_solve, lp, ls, lw, ty, to, tf, T.mp, td, ts, tl,
                                       *reinterpret_cast<FusedShared<16>*>(&sh));
             break;
         case 32:
-            analysis_body<32, PASSES>(bx, T.nb_solve, lp, ls, lw, ty, to, tf, T.mp, td, ts,
+            analysis_body<32, PASSES>(bx, T.nb_solve, lp, ls, lw, ty, to, tf, T.mp, td, ts, tl,
                                       *reinterpret_cast<FusedShared<32>*>(&sh));
             break;
-        default: analysis_body<64, PASSES>(bx, T.nb_solve, lp, ls, lw, ty, to, tf, T.mp, td, ts, sh); break;
+        default: analysis_body<64, PASSES>(bx, T.nb_solve, lp, ls, lw, ty, to, tf, T.mp, td, ts, tl, sh); break;
     }
 }
 
@@ -1646,10 +1781,16 @@ MixedParams mixed_params(const Ctx& c, unsigned long long* sweeps32, unsigned lo
     mp.sweeps64 = sweeps64;
     mp.chain = c.mix_chain;
     mp.write_state = 1;
+    mp.series = c.d_series;
+    mp.series_scale = std::exp2(-float(std::ilogb(mp.diag)));
+    mp.series_steps = c.prof ? c.d_series_steps : nullptr;
     return mp;
 }
 
 }  // namespace
+
+size_t series_table_bytes() { return series_table().size() * sizeof(float); }
+const float* series_table_host() { return series_table().data(); }
 
 int mixed_width(int M) {
     int N = 16;
@@ -1669,16 +1810,18 @@ hipError_t launch_letkf_mixed(Ctx& c, float* f, unsigned long long* sweeps32, un
     if (c.mix_width != N || c.mix_chain < 1) return hipErrorInvalidValue;
     MixedParams mp = mixed_params(c, sweeps32, sweeps64);
     if (mixed_fused(c)) {
-        // one kernel, no workspace
-        const long long nb = mixed_fused_blocks(c.nx, c.ny, mp.chain);
+        // the series, then the sweeps for what it left
+        if (!c.d_left || !c.d_series) return hipErrorInvalidValue;
         if (solve_only) {
             mp.write_state = 0;
             mp.dump_n = 0;
         }
-        const dim3 grid_a{unsigned(nb), 1u, 1u};
+        const dim3 grid_s{unsigned((c.nodes + 7) / 8 * 8)}, grid_a{unsigned(mixed_fused_blocks(c.nx, c.ny, mp.chain))};
 #define LAUNCH_FUSED(NN, PP)                                                                                   \
+    k_series_analysis<NN, PP><<<grid_s, dim3(64), 0, c.stream>>>(c.d_loc_ptr, c.d_loc_site, c.d_loc_w, c.d_dy, \
+                                                                 c.d_dyo, f, mp, c.d_status, c.d_left);        \
     k_mixed_analysis<NN, PP><<<grid_a, dim3(64), 0, c.stream>>>(c.d_loc_ptr, c.d_loc_site, c.d_loc_w, c.d_dy,  \
-                                                                c.d_dyo, f, mp, c.d_dump, c.d_status)
+                                                                c.d_dyo, f, mp, c.d_dump, c.d_status, c.d_left)
         switch (N * 10 + (passes == 3 ? 3 : 1)) {
             case 163: LAUNCH_FUSED(16, 3); break;
             case 161: LAUNCH_FUSED(16, 1); break;
@@ -1743,7 +1886,7 @@ hipError_t launch_letkf_mixed_group(Ctx* const* cs, int n, hipStream_t stream) {
         const int N = mixed_width(c.M);
         if (!c.d_loc_ptr || !c.d_dy || !c.d_dyo || c.mix_width != N || (c.dump_n > 0 && !c.d_dump))
             return hipErrorInvalidValue;
-        if (sweep64 && (!c.d_mix_u || !c.d_mix_b)) return hipErrorInvalidValue;
+        if (sweep64 ? (!c.d_mix_u || !c.d_mix_b) : (!c.d_left || !c.d_series)) return hipErrorInvalidValue;
         if (c.cfg.gram_passes != passes || (c.cfg.jacobi_fp64_sweeps > 0) != sweep64) return hipErrorInvalidValue;
         MixedTask& T = G.t[k];
         T.loc_ptr = c.d_loc_ptr;
@@ -1756,6 +1899,7 @@ hipError_t launch_letkf_mixed_group(Ctx* const* cs, int n, hipStream_t stream) {
         T.f = c.f[c.cur];
         T.dump = c.d_dump;
         T.status = c.d_status;
+        T.left = c.d_left;
         T.mp = mixed_params(c, nullptr, nullptr);
         T.N = N;
         const long long chains = sweep64 ? (c.nodes + T.mp.chain - 1) / T.mp.chain
@@ -1769,6 +1913,12 @@ hipError_t launch_letkf_mixed_group(Ctx* const* cs, int n, hipStream_t stream) {
     }
     if (bs > (1LL << 31) - 1 || bf > (1LL << 31) - 1) return hipErrorInvalidValue;
     if (!sweep64) {
+        if (passes == 3)
+            k_series_analysis_group<3><<<unsigned(bf), 64, 0, stream>>>(G);
+        else
+            k_series_analysis_group<1><<<unsigned(bf), 64, 0, stream>>>(G);
+        const hipError_t es = hipGetLastError();
+        if (es != hipSuccess) return es;
         if (passes == 3)
             k_mixed_analysis_group<3><<<unsigned(bs), 64, 0, stream>>>(G);
         else
