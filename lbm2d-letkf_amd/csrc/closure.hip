@@ -8,9 +8,9 @@
 // model tau_dev = -2 nu_t S_dev(u_bar): loss = w ((2 nu a + t1)^2 + (2 nu b + t2)^2)
 // with (a, b) the deviatoric strain of u_bar and t1 = (tau11 - tau22)/2, t2 = tau12.
 //
-// Training kernels run in FP32 on the vector ALU: one sample per lane, the
-// parameters in LDS (broadcast reads), per-workgroup partial gradients summed in a
-// fixed order (deterministic), then Adam.
+// Training kernels run in FP32, the products on the matrix cores, 16 samples per
+// wavefront at a time; per-workgroup partial gradients are summed in a fixed order
+// (deterministic), then Adam.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -26,14 +26,13 @@ namespace lbmletkf {
 
 namespace {
 
-__device__ __forceinline__ float gelu_f(float x) {
+// gelu(x) = x/2 (1 + tanh(w)), w = k (x + 0.044715 x^3), and its derivative, by
+// (1 + tanh(w))/2 = 1/(1 + exp(-2 w)): no cancellation at either end
+__device__ __forceinline__ void gelu_f(float x, float& h, float& d) {
     const float k = 0.7978845608028654f;  // sqrt(2/pi)
-    return 0.5f * x * (1.f + tanhf(k * (x + 0.044715f * x * x * x)));
-}
-__device__ __forceinline__ float gelu_df(float x) {
-    const float k = 0.7978845608028654f;
-    const float t = tanhf(k * (x + 0.044715f * x * x * x));
-    return 0.5f * (1.f + t) + 0.5f * x * (1.f - t * t) * k * (1.f + 3.f * 0.044715f * x * x);
+    const float s = 1.f / (1.f + expf(-2.f * k * (x + 0.044715f * x * x * x)));
+    h = x * s;
+    d = s + 2.f * h * (1.f - s) * k * (1.f + 3.f * 0.044715f * x * x);
 }
 __device__ __forceinline__ float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.f / (1.f + expf(-z)); }
@@ -118,131 +117,294 @@ __global__ void k_closure_samples(const float* __restrict__ fields, int nx, int 
 }
 
 // ---- training ------------------------------------------------------------------
-constexpr int TB = 64;  // samples (lanes) per workgroup
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int TB = 256;             // threads of a gradient workgroup: four wavefronts
+constexpr int TG = 16;              // samples a wavefront takes at a time
+constexpr int GRAD_BLOCKS = 512;    // at most: two wavefronts per SIMD
+constexpr int WLD = CL_H + 4;       // row stride of the LDS arrays (16-byte rows, spread over the banks)
+constexpr int W1LD = 21;            // row stride of the first layer's weights in LDS
 constexpr int PST = CL_NPARAM + 1;  // partial record: gradient + loss
 
-// Loss and gradient of `count` samples starting at `first` (through the
-// permutation idx = (pa * k + pc) mod n_total when permute != 0); each workgroup
-// writes its partial sums to partial[blockIdx.x][0..CL_NPARAM].
-__global__ __launch_bounds__(TB) void k_closure_grad(const float* __restrict__ params,
-                                                     const float* __restrict__ samples, long long n_total,
-                                                     long long first, long long count, unsigned long long pa,
-                                                     unsigned long long pc, int permute, float nu_scale, float w_norm,
-                                                     float* __restrict__ partial) {
-    __shared__ float P[CL_NPARAM];
-    __shared__ float sx[TB][CL_IN + 1];
-    __shared__ float sh1[TB][CL_H + 1];
-    __shared__ float sdp1[TB][CL_H + 1];
-    __shared__ float sdp2[TB][CL_H + 1];
-    __shared__ float sh2[TB][CL_H + 1];
-    __shared__ float sdz[TB], sloss[TB];
-    const int t = threadIdx.x;
-    for (int k = t; k < CL_NPARAM; k += TB) P[k] = params[k];
+// LDS writes of this wavefront before reads by its other lanes
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// x summed over the 16 lanes of its row (the samples)
+__device__ __forceinline__ float row_sum(float x) {
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off);
+    return x;
+}
+
+// x summed over the four lane groups
+__device__ __forceinline__ float group_sum(float x) {
+    x += __shfl_xor(x, 16);
+    return x + __shfl_xor(x, 32);
+}
+
+// Loss and gradient of `count` samples starting at `first` (through the permutation
+// idx = (pa * k + pc) mod n_total when permute != 0); each workgroup writes its partial
+// sums to partial[blockIdx.x][0..CL_NPARAM].
+//
+// A wavefront steps through groups of 16 samples, every product on the FP32 matrix cores
+// (v_mfma_f32_16x16x4f32: A[m][k] from lane (m = lane % 16, k = lane / 16), B[k][n] from
+// lane (n = lane % 16, k = lane / 16), D[4 (lane / 16) + r][lane % 16]).  Forward and back
+// through the layers the hidden units are rows and the samples columns: lane (c, g) holds
+// units 16 T + 4 g + r of sample c, and those accumulators are the next product's B
+// operand with the sum over k in the order (T, g, r).  The weight gradients sum over the
+// samples, so there the samples are rows: h1, dp1 and dp2 pass through LDS once to be
+// turned.  Bound by the matrix cores and the 128 tanhf of a sample; 200,000 samples take
+// 125 us (1210 us with one sample per lane on the vector ALU, whose weights come
+// from LDS one broadcast per multiply-add).
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(2))) void k_closure_grad(
+    const float* __restrict__ params, const float* __restrict__ samples, long long n_total, long long first,
+    long long count, unsigned long long pa, unsigned long long pc, int permute, float nu_scale, float w_norm,
+    float* __restrict__ partial) {
+    __shared__ __align__(16) float lds[CL_H * WLD + (TB / 64) * TG * WLD];
+    __shared__ __align__(16) float sb[3][CL_H];  // b1, b2, w3
+    __shared__ float w1[CL_H * W1LD];            // inputs 18, 19 zero
+    static_assert(sizeof(lds) >= PST * sizeof(float), "the partial sums reuse the arrays");
+    float* w2 = lds;
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int c = lane % 16, g = lane / 16;
+    float* turn = lds + CL_H * WLD + wave * TG * WLD;  // [sample][unit]
+    for (int k = threadIdx.x; k < CL_H * CL_H; k += TB) w2[(k / CL_H) * WLD + k % CL_H] = params[CL_W2 + k];
+    for (int k = threadIdx.x; k < CL_H; k += TB) {
+        sb[0][k] = params[CL_B1 + k];
+        sb[1][k] = params[CL_B2 + k];
+        sb[2][k] = params[CL_W3 + k];
+    }
+    // first layer: lane group g holds inputs 5 g .. 5 g + 4 (18 of 20)
+    for (int k = threadIdx.x; k < CL_H * W1LD; k += TB)
+        w1[k] = k % W1LD < CL_IN ? params[CL_W1 + (k / W1LD) * CL_IN + k % W1LD] : 0.f;
+    const float b3 = params[CL_B3];
     __syncthreads();
 
-    const long long k = first + (long long)blockIdx.x * TB + t;
-    const bool valid = k < first + count;
-    long long idx = k;
-    if (permute) idx = (long long)((pa * (unsigned long long)k + pc) % (unsigned long long)n_total);
-    if (!valid) idx = 0;
-    const float* smp = samples + idx * CL_SAMPLE;
-    float x[CL_IN];
+    auto vec = [&](int a, int I, int g) { return *reinterpret_cast<const f32x4*>(&sb[a][16 * I + 4 * g]); };
+    // values (units x samples) as samples x units: t[T][r] = unit 16 T + c of sample 4 g + r
+    auto turned = [&](const f32x4 (&v)[4], f32x4 (&t)[4], int c, int g) {
+        wave_sync();  // the last reads are done
 #pragma unroll
-    for (int i = 0; i < CL_IN; ++i) x[i] = smp[i];
-    const float a = smp[18], b = smp[19], t1 = smp[20], t2 = smp[21];
+        for (int T = 0; T < 4; ++T) *reinterpret_cast<f32x4*>(&turn[c * WLD + 16 * T + 4 * g]) = v[T];
+        wave_sync();
+#pragma unroll
+        for (int T = 0; T < 4; ++T)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) t[T][r] = turn[(4 * g + r) * WLD + 16 * T + c];
+    };
+    f32x4 gw2[4][4], gw1[4][2];
+    float gb2[4], gw3[4];  // of unit 16 T + c, the samples of this lane group
+#pragma unroll
+    for (int I = 0; I < 4; ++I) {
+        gb2[I] = gw3[I] = 0.f;
+        gw1[I][0] = gw1[I][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int J = 0; J < 4; ++J) gw2[I][J] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    float gb3 = 0.f, loss = 0.f;
+    const long long groups = (count + TG - 1) / TG;
+    for (long long grp = (long long)blockIdx.x * (TB / 64) + wave; grp < groups;
+         grp += (long long)gridDim.x * (TB / 64)) {
+        // from an opaque copy: the bias vectors and LDS addresses are formed in the loop, not
+        // held across it beside the gradient sums
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int c = ln % 16, g = ln / 16;
+        const long long k = first + grp * TG + c;
+        const bool valid = k < first + count;
+        long long idx = k;
+        if (permute) idx = (long long)((pa * (unsigned long long)k + pc) % (unsigned long long)n_total);
+        if (!valid) idx = 0;
+        const float* smp = samples + idx * CL_SAMPLE;
+        float x[5];
+#pragma unroll
+        for (int s = 0; s < 5; ++s) x[s] = 5 * g + s < CL_IN ? smp[5 * g + s] : (5 * g + s == CL_IN ? 1.f : 0.f);
+        const float a = smp[18], b = smp[19], t1 = smp[20], t2 = smp[21];
 
-    // forward; sdp1/sdp2 first hold gelu'(p1), gelu'(p2)
-    for (int o = 0; o < CL_H; ++o) {
-        float s = P[CL_B1 + o];
+        // forward
+        f32x4 h1[4], d1[4];
 #pragma unroll
-        for (int i = 0; i < CL_IN; ++i) s = fmaf(P[CL_W1 + o * CL_IN + i], x[i], s);
-        sh1[t][o] = gelu_f(s);
-        sdp1[t][o] = gelu_df(s);
-    }
-    float z = P[CL_B3];
-    for (int o = 0; o < CL_H; ++o) {
-        float s = P[CL_B2 + o];
-        for (int i = 0; i < CL_H; ++i) s = fmaf(P[CL_W2 + o * CL_H + i], sh1[t][i], s);
-        const float h = gelu_f(s);
-        sh2[t][o] = h;
-        sdp2[t][o] = gelu_df(s);
-        z = fmaf(P[CL_W3 + o], h, z);
-    }
-    const float nu = nu_scale * softplus_f(z);
-    const float r1 = 2.f * nu * a + t1, r2 = 2.f * nu * b + t2;
-    sloss[t] = valid ? w_norm * (r1 * r1 + r2 * r2) : 0.f;
-    const float dz = valid ? w_norm * 4.f * (r1 * a + r2 * b) * nu_scale * sigmoid_f(z) : 0.f;
-    sdz[t] = dz;
+        for (int I = 0; I < 4; ++I) {
+            f32x4 p = vec(0, I, g);
+#pragma unroll
+            for (int s = 0; s < 5; ++s) p = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[(16 * I + c) * W1LD + 5 * g + s], x[s], p, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float h, d;
+                gelu_f(p[r], h, d);
+                h1[I][r] = h;
+                d1[I][r] = d;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        f32x4 p2[4];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) p2[I] = vec(1, I, g);
+#pragma unroll
+        for (int T = 0; T < 4; ++T)
+#pragma unroll
+            for (int I = 0; I < 4; ++I) {
+                const f32x4 w = *reinterpret_cast<const f32x4*>(&w2[(16 * I + c) * WLD + 16 * T + 4 * g]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p2[I] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[r], h1[T][r], p2[I], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        float z = 0.f;
+        f32x4 h2[4], dp2[4];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            const f32x4 w3 = vec(2, I, g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float h, d;
+                gelu_f(p2[I][r], h, d);
+                z = fmaf(w3[r], h, z);
+                h2[I][r] = h;
+                dp2[I][r] = w3[r] * d;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        z = group_sum(z) + b3;
+        const float nu = nu_scale * softplus_f(z);
+        const float r1 = 2.f * nu * a + t1, r2 = 2.f * nu * b + t2;
+        const float dz = valid ? w_norm * 4.f * (r1 * a + r2 * b) * nu_scale * sigmoid_f(z) : 0.f;
+        if (g == 0) {
+            loss += valid ? w_norm * (r1 * r1 + r2 * r2) : 0.f;
+            gb3 += dz;
+        }
+        // backward to the hidden layers
+        f32x4 dp1[4];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                h2[I][r] *= dz;
+                dp2[I][r] *= dz;
+            }
+            dp1[I] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int T = 0; T < 4; ++T)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                for (int I = 0; I < 4; ++I)
+                    dp1[I] = __builtin_amdgcn_mfma_f32_16x16x4f32(w2[(16 * T + 4 * g + r) * WLD + 16 * I + c], dp2[T][r],
+                                                                  dp1[I], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+        for (int I = 0; I < 4; ++I) dp1[I] *= d1[I];
 
-    // backward to the hidden layers
-    float dh1[CL_H];
+        // parameter gradients: sums over the samples
+        f32x4 ht[4], dt[4];
+        turned(h2, dt, c, g);
 #pragma unroll
-    for (int i = 0; i < CL_H; ++i) dh1[i] = 0.f;
-    for (int o = 0; o < CL_H; ++o) {
-        const float dp2 = dz * P[CL_W3 + o] * sdp2[t][o];
-        sdp2[t][o] = dp2;
+        for (int T = 0; T < 4; ++T) gw3[T] += (dt[T][0] + dt[T][1]) + (dt[T][2] + dt[T][3]);
+        turned(h1, ht, c, g);
+        turned(dp2, dt, c, g);
 #pragma unroll
-        for (int i = 0; i < CL_H; ++i) dh1[i] = fmaf(P[CL_W2 + o * CL_H + i], dp2, dh1[i]);
+        for (int T = 0; T < 4; ++T) gb2[T] += (dt[T][0] + dt[T][1]) + (dt[T][2] + dt[T][3]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int O = 0; O < 4; ++O)
+#pragma unroll
+                for (int I = 0; I < 4; ++I)
+                    gw2[O][I] = __builtin_amdgcn_mfma_f32_16x16x4f32(dt[O][r], ht[I][r], gw2[O][I], 0, 0, 0);
+        turned(dp1, dt, c, g);
+        wave_sync();
+#pragma unroll
+        for (int s = 0; s < 5; ++s) turn[c * WLD + 5 * g + s] = x[s];
+        wave_sync();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float x0 = turn[(4 * g + r) * WLD + c], x1 = c < 4 ? turn[(4 * g + r) * WLD + 16 + c] : 0.f;
+#pragma unroll
+            for (int O = 0; O < 4; ++O) {
+                gw1[O][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(dt[O][r], x0, gw1[O][0], 0, 0, 0);
+                gw1[O][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(dt[O][r], x1, gw1[O][1], 0, 0, 0);
+            }
+        }
     }
+    // the four wavefronts' sums in turn; input 18 is constant one: its gradient is b1's
+    gb3 = row_sum(gb3);
+    loss = row_sum(loss);
+    float* out = lds;
+    for (int w = 0; w < TB / 64; ++w) {
+        __syncthreads();
+        if (wave != w) continue;
+        auto put = [&](int p, float v) { out[p] = w == 0 ? v : out[p] + v; };
 #pragma unroll
-    for (int i = 0; i < CL_H; ++i) sdp1[t][i] *= dh1[i];
+        for (int O = 0; O < 4; ++O)
 #pragma unroll
-    for (int i = 0; i < CL_IN; ++i) sx[t][i] = x[i];
+            for (int r = 0; r < 4; ++r) {
+                const int o = 16 * O + 4 * g + r;
+#pragma unroll
+                for (int I = 0; I < 4; ++I) put(CL_W2 + o * CL_H + 16 * I + c, gw2[O][I][r]);
+                put(CL_W1 + o * CL_IN + c, gw1[O][0][r]);
+                if (c < 2) put(CL_W1 + o * CL_IN + 16 + c, gw1[O][1][r]);
+                if (c == 2) put(CL_B1 + o, gw1[O][1][r]);
+            }
+#pragma unroll
+        for (int T = 0; T < 4; ++T) {
+            const float s2 = group_sum(gb2[T]), s3 = group_sum(gw3[T]);
+            if (g == 0) {
+                put(CL_B2 + 16 * T + c, s2);
+                put(CL_W3 + 16 * T + c, s3);
+            }
+        }
+        if (lane == 0) {
+            put(CL_B3, gb3);
+            put(CL_NPARAM, loss);
+        }
+    }
     __syncthreads();
-
-    // parameter gradients: lane o owns row o of W1 and W2, b1[o], b2[o], w3[o]
-    const int o = t;
-    float gw2[CL_H], gw1[CL_IN];
-#pragma unroll
-    for (int i = 0; i < CL_H; ++i) gw2[i] = 0.f;
-#pragma unroll
-    for (int i = 0; i < CL_IN; ++i) gw1[i] = 0.f;
-    float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, loss = 0.f;
-    for (int s = 0; s < TB; ++s) {
-        const float d2 = sdp2[s][o], d1 = sdp1[s][o];
-#pragma unroll
-        for (int i = 0; i < CL_H; ++i) gw2[i] = fmaf(d2, sh1[s][i], gw2[i]);
-#pragma unroll
-        for (int i = 0; i < CL_IN; ++i) gw1[i] = fmaf(d1, sx[s][i], gw1[i]);
-        gb1 += d1;
-        gb2 += d2;
-        gw3 = fmaf(sdz[s], sh2[s][o], gw3);
-        gb3 += sdz[s];
-        loss += sloss[s];
-    }
     float* pr = partial + (long long)blockIdx.x * PST;
-#pragma unroll
-    for (int i = 0; i < CL_H; ++i) pr[CL_W2 + o * CL_H + i] = gw2[i];
-#pragma unroll
-    for (int i = 0; i < CL_IN; ++i) pr[CL_W1 + o * CL_IN + i] = gw1[i];
-    pr[CL_B1 + o] = gb1;
-    pr[CL_B2 + o] = gb2;
-    pr[CL_W3 + o] = gw3;
-    if (o == 0) {
-        pr[CL_B3] = gb3;
-        pr[CL_NPARAM] = loss;
-    }
+    for (int k = threadIdx.x; k < PST; k += TB) pr[k] = out[k];
 }
 
-// grad[p] = sum over workgroups (in order) / count; out[CL_NPARAM] = mean loss
-__global__ void k_closure_reduce(const float* __restrict__ partial, int nb, float inv_count, float* __restrict__ out) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > CL_NPARAM) return;
+// grad[p] = sum over workgroups / count, out[CL_NPARAM] = mean loss: 64 parameters per
+// workgroup, RED_ROWS threads each a fixed share of the workgroups, summed in FP64 in a
+// fixed order.  ADAM: one Adam update of the parameters with that gradient, the loss to
+// *hist (may be null).
+constexpr int RED_ROWS = 16;
+struct AdamParams {
+    float *params, *m, *v, *hist;
+    float lr, b1, b2, eps, c1, c2;
+};
+template <bool ADAM>
+__global__ __launch_bounds__(64 * RED_ROWS) void k_closure_reduce(const float* __restrict__ partial, int nb,
+                                                                  float inv_count, float* __restrict__ out,
+                                                                  AdamParams ad) {
+    __shared__ double sum[RED_ROWS][64];
+    const int t = threadIdx.x % 64, row = threadIdx.x / 64;
+    const int p = blockIdx.x * 64 + t;
     double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += partial[(long long)b * PST + p];
-    out[p] = float(s * inv_count);
-}
-
-__global__ void k_adam(float* __restrict__ params, const float* __restrict__ grad, float* __restrict__ m,
-                       float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= CL_NPARAM) return;
-    const float g = grad[p];
-    const float mm = b1 * m[p] + (1.f - b1) * g;
-    const float vv = b2 * v[p] + (1.f - b2) * g * g;
-    m[p] = mm;
-    v[p] = vv;
-    params[p] -= lr * (mm * c1) / (sqrtf(vv * c2) + eps);
+    if (p < PST)
+        for (int b = row; b < nb; b += RED_ROWS) s += partial[(long long)b * PST + p];
+    sum[row][t] = s;
+    __syncthreads();
+    if (row > 0 || p >= PST) return;
+#pragma unroll
+    for (int r = 1; r < RED_ROWS; ++r) s += sum[r][t];
+    const float gr = float(s * inv_count);
+    out[p] = gr;
+    if constexpr (ADAM) {
+        if (p == CL_NPARAM) {
+            if (ad.hist) *ad.hist = gr;
+            return;
+        }
+        const float mm = ad.b1 * ad.m[p] + (1.f - ad.b1) * gr;
+        const float vv = ad.b2 * ad.v[p] + (1.f - ad.b2) * gr * gr;
+        ad.m[p] = mm;
+        ad.v[p] = vv;
+        ad.params[p] -= ad.lr * (mm * ad.c1) / (sqrtf(vv * ad.c2) + ad.eps);
+    }
 }
 
 // mean of t1^2 + t2^2 over the samples (per-workgroup partial sums in FP64)
@@ -266,7 +428,6 @@ __global__ void k_target_power(const float* __restrict__ samples, long long n, d
 using namespace lbmnode;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int MX = 64, MY = 16, MNT = 256;   // tile of one member, threads per workgroup
 constexpr int MROWS = MNT / MX;              // 4 rows per pass
@@ -591,20 +752,27 @@ int coarse_fields(Trainer* t, Ctx* fine, int member, int F, long long& nc, int& 
     return LBMLETKF_OK;
 }
 
+// Loss and gradient into d_grad; with `adam` one update of the parameters too.
 int grad_launch(Trainer* t, long long first, long long count, bool permute, unsigned long long pa,
-                unsigned long long pc, float w_norm) {
-    const int nb = int((count + TB - 1) / TB);
+                unsigned long long pc, float w_norm, const AdamParams* adam = nullptr) {
+    const long long groups = (count + TG - 1) / TG;
+    const int nb = int(std::min<long long>(GRAD_BLOCKS, (groups + TB / 64 - 1) / (TB / 64)));
     if (nb > t->max_blocks) {
         if (t->d_partial) TR_TRY(hipFree(t->d_partial));
         t->d_partial = nullptr;
+        t->max_blocks = 0;
         TR_TRY(hipMalloc(&t->d_partial, sizeof(float) * (size_t)nb * PST));
         t->max_blocks = nb;
     }
     k_closure_grad<<<nb, TB, 0, t->stream>>>(t->d_params, t->d_samples, t->n, first, count, pa, pc, permute ? 1 : 0,
                                              float(t->cfg.closure_nu_scale), w_norm, t->d_partial);
     TR_TRY(hipGetLastError());
-    k_closure_reduce<<<(CL_NPARAM + 1 + 255) / 256, 256, 0, t->stream>>>(t->d_partial, nb, float(1.0 / double(count)),
-                                                                        t->d_grad);
+    const int rb = (PST + 63) / 64;
+    const float inv = float(1.0 / double(count));
+    if (adam)
+        k_closure_reduce<true><<<rb, 64 * RED_ROWS, 0, t->stream>>>(t->d_partial, nb, inv, t->d_grad, *adam);
+    else
+        k_closure_reduce<false><<<rb, 64 * RED_ROWS, 0, t->stream>>>(t->d_partial, nb, inv, t->d_grad, AdamParams{});
     TR_TRY(hipGetLastError());
     return LBMLETKF_OK;
 }
@@ -791,17 +959,11 @@ int lbmletkf_trainer_train(lbmletkf_trainer* tr, int batch, int steps, double lr
         unsigned long long pa = primes[epoch % 8];
         while (std::gcd(pa, (unsigned long long)t->n) != 1) pa += 2;
         const unsigned long long pc = (unsigned long long)(epoch * 7919 + 17) % (unsigned long long)t->n;
-        st = grad_launch(t, pos, batch, true, pa % (unsigned long long)t->n, pc, wn);
-        if (st != LBMLETKF_OK) break;
-        ++t->adam_t;
-        const float c1 = float(1.0 / (1.0 - std::pow(b1, double(t->adam_t))));
-        const float c2 = float(1.0 / (1.0 - std::pow(b2, double(t->adam_t))));
-        k_adam<<<(CL_NPARAM + 255) / 256, 256, 0, t->stream>>>(t->d_params, t->d_grad, t->d_m, t->d_v, float(lr),
-                                                               float(b1), float(b2), float(eps), c1, c2);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess && d_hist)
-            e = hipMemcpyAsync(d_hist + s, t->d_grad + CL_NPARAM, sizeof(float), hipMemcpyDeviceToDevice, t->stream);
-        if (e != hipSuccess) st = report_error(nullptr, LBMLETKF_ERR_HIP, std::string("train: ") + hipGetErrorString(e));
+        AdamParams ad{t->d_params, t->d_m, t->d_v, d_hist ? d_hist + s : nullptr, float(lr), float(b1), float(b2), float(eps)};
+        ad.c1 = float(1.0 / (1.0 - std::pow(b1, double(t->adam_t + 1))));
+        ad.c2 = float(1.0 / (1.0 - std::pow(b2, double(t->adam_t + 1))));
+        st = grad_launch(t, pos, batch, true, pa % (unsigned long long)t->n, pc, wn, &ad);
+        if (st == LBMLETKF_OK) ++t->adam_t;
     }
     hipError_t e = hipStreamSynchronize(t->stream);
     if (e == hipSuccess && d_hist && st == LBMLETKF_OK)
