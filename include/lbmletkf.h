@@ -51,7 +51,7 @@ extern "C" {
 #define LBMLETKF_CLOSURE_MLP         1
 
 /* analysis variants */
-#define LBMLETKF_VARIANT_PLAIN       0   /* FP32 Gram on VALU, FP64 Jacobi */
+#define LBMLETKF_VARIANT_PLAIN       0   /* FP32 Gram matrix, FP64 solve */
 #define LBMLETKF_VARIANT_MIXED       1   /* fused LETKF, mixed precision; cycles replayed as graphs */
 
 /* All physical / numerical parameters of a run.  The reference fixes these at
@@ -91,7 +91,7 @@ typedef struct lbmletkf_config {
     double inflation;           /* LETKF_COVINF beta (config.h:48-50)                       */
     int    da_interval;         /* LBM steps per DA cycle (iiter*DAPRUNE, config.h:136,142) */
     int    variant;             /* LBMLETKF_VARIANT_*                                       */
-    double jacobi_tol;          /* relative off-diagonal tolerance of the eigensolver       */
+    double jacobi_tol;          /* relative off-diagonal tolerance of the eigensolver (where one is taken: a local problem of condition above 65500 (PLAIN) or 1023 (MIXED), a dumped gridpoint) */
     int    jacobi_max_sweeps;   /* cusolver syevj uses tol 1e-6, 100 sweeps (cu_matrix_eigensolver_wrapper.hpp:192-193) */
     int    gram_passes;         /* MIXED: 1 = bf16 operands, 3 = split bf16 (hi*hi + hi*lo + lo*hi) */
     int    jacobi_fp64_sweeps;  /* MIXED: at most this many FP64 sweeps after the FP32 phase (presets: 0) */

@@ -350,6 +350,10 @@ int setup_obs_impl(Ctx* c) {
 
 int ensure_plain_buffers(Ctx* c) {
     if (c->d_gram) return LBMLETKF_OK;
+    const std::vector<double>& t = series_table64();
+    HIP_TRY(c, hipMalloc(&c->d_series64, t.size() * sizeof(double)));
+    HIP_TRY(c, hipMemcpy(c->d_series64, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
+    HIP_TRY(c, dalloc(&c->d_left, c->nodes));
     HIP_TRY(c, dalloc(&c->d_gram, (size_t)c->nodes * c->M * c->M));
     HIP_TRY(c, dalloc(&c->d_bvec, (size_t)c->nodes * c->M));
     return LBMLETKF_OK;
@@ -364,8 +368,9 @@ int ensure_mixed_buffers(Ctx* c) {
         HIP_TRY(c, dalloc(&c->d_mix_b, (size_t)c->nodes * N));
     }
     if (mixed_fused(*c) && !c->d_series) {
-        HIP_TRY(c, hipMalloc(&c->d_series, series_table_bytes()));
-        HIP_TRY(c, hipMemcpy(c->d_series, series_table_host(), series_table_bytes(), hipMemcpyHostToDevice));
+        const std::vector<float>& t = series_table32();
+        HIP_TRY(c, hipMalloc(&c->d_series, t.size() * sizeof(float)));
+        HIP_TRY(c, hipMemcpy(c->d_series, t.data(), t.size() * sizeof(float), hipMemcpyHostToDevice));
         HIP_TRY(c, dalloc(&c->d_left, c->nodes));
     }
     c->mix_width = N;
@@ -510,6 +515,9 @@ int analysis_launches(Ctx* c) {
         c->dump_kind = 1;
         return LBMLETKF_OK;
     }
+    hipEvent_t e3 = prof_begin(c);
+    HIP_TRY(c, launch_series_fp64(*c, c->f[c->cur]));
+    prof_end(c, PH_SOLVE, e3, 1, 0);
     hipEvent_t e1 = prof_begin(c);
     HIP_TRY(c, launch_gram_fp32(*c));
     prof_end(c, PH_GRAM, e1, 1, c->obs.n_entries * c->obs.n_vars);
@@ -577,7 +585,7 @@ Ctx::~Ctx() {
     void* ptrs[] = {f[0], f[1], force_xy, d_force_draws, d_force_table, d_force, d_step, d_status,
                     d_site_node, d_loc_ptr, d_loc_site, d_loc_w, d_obs_coef, d_yo, d_hx, d_hx1, d_dy,
                     d_dyo, d_gram, d_bvec, d_mix_u, d_mix_b, d_dump, d_red, d_truth, d_sweeps,
-                    d_sweeps64, d_series_steps, d_closure, d_series, d_left, d_site_map, d_ens_uv, d_ens_out};
+                    d_sweeps64, d_series_steps, d_closure, d_series, d_series64, d_left, d_site_map, d_ens_uv, d_ens_out};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (const ProfRec& r : prof_pending) {

@@ -120,7 +120,8 @@ struct Ctx {
     float* d_mix_b = nullptr;     // [nodes][N] b = dY^T R^-1 dyo
     int mix_width = 0;
     float4* d_series = nullptr;   // coefficients of the fused form's series (letkf_series.hpp)
-    unsigned char* d_left = nullptr;  // [nodes] gridpoints the series left to the sweeps
+    double4* d_series64 = nullptr;    // and of the PLAIN variant's
+    unsigned char* d_left = nullptr;  // [nodes] gridpoints the series left to the eigensolve
     int mix_chain = 8;            // consecutive gridpoints per wavefront in k_mixed_solve
     // shape of the LBM step: 1 the rule of lbm.hip on the grid and ensemble size (blocks
     // or strips), k > 1 tiles of 64x16 per workgroup (k_lbm_fused),
@@ -232,14 +233,18 @@ hipError_t launch_obs_moments(Ctx& c, const float* f, double* hx, int member0, i
 hipError_t launch_obs_prepare(Ctx& c);
 hipError_t launch_observe(Ctx& c, const double* hx_member, float* yo, uint64_t seed,
                           uint64_t counter, int noise);
+// The PLAIN analysis: the series in FP64, then C and b, and the eigensolve, of the
+// gridpoints it left (Ctx::d_left)
+hipError_t launch_series_fp64(Ctx& c, float* f);
+// the coefficient table of its series, for Ctx::d_series64
+const std::vector<double>& series_table64();
 hipError_t launch_gram_fp32(Ctx& c);
 hipError_t launch_solve_fp64(Ctx& c, float* f, unsigned long long* sweeps);
 
 // ---- launchers (letkf_mixed.hip) ----------------------------------------------
 int mixed_width(int M);
 // the coefficient table of the fused form's series, for Ctx::d_series
-size_t series_table_bytes();
-const float* series_table_host();
+const std::vector<float>& series_table32();
 // the presets' form: one fused kernel (no FP64 sweeps requested)
 bool mixed_fused(const Ctx& c);
 long long mixed_fused_blocks(int nx, int ny, int chain);

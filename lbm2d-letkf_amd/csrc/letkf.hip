@@ -15,6 +15,7 @@
 // instead re-packs a dense window per gridpoint (src/letkf.cu:150-187) and moves
 // it between ranks with all-to-alls.
 #include "context.hpp"
+#include "letkf_series.hpp"
 #include "philox.hpp"
 
 namespace lbmletkf {
@@ -203,81 +204,229 @@ __global__ void k_observe(const double* __restrict__ hx, float* __restrict__ yo,
 // Replaces the two strided-batched GEMMs of src/util/letkf_solver.h:251-254
 // (the reference multiplies by a dense diagonal rR first).
 // ----------------------------------------------------------------------------
-constexpr int GRAM_NT = 256, GRAM_CH = 32, GRAM_MP = 64;
+constexpr int GRAM_NT = 256, GRAM_CH = 32, GRAM_MP = 64, GRAM_RUN = 16;
 
 __global__ __launch_bounds__(GRAM_NT) void k_gram_fp32(
     const int* __restrict__ loc_ptr, const int* __restrict__ loc_site,
     const float* __restrict__ loc_w, const float* __restrict__ dy, const float* __restrict__ dyo,
     const float* __restrict__ coef, int n_vars, int M, float diag, float* __restrict__ gram,
-    float* __restrict__ bvec) {
+    float* __restrict__ bvec, const unsigned char* __restrict__ left, int nodes) {
     __shared__ float sD[GRAM_CH][GRAM_MP];
     __shared__ float sW[GRAM_CH], sE[GRAM_CH];
-    const int g = blockIdx.x;
     const int t = threadIdx.x;
     const int NB = (M + 3) / 4;
     const bool active = t < NB * NB;
     const int kb = t % NB, lb = t / NB;
-    float acc[4][4] = {};
-    float bacc[4] = {};
-    const int e0 = loc_ptr[g], e1 = loc_ptr[g + 1];
-    const int total = (e1 - e0) * n_vars;
-    for (int base = 0; base < total; base += GRAM_CH) {
-        for (int idx = t; idx < GRAM_CH * GRAM_MP; idx += GRAM_NT) {
-            const int r = idx / GRAM_MP, k = idx % GRAM_MP;
-            const int fi = base + r;
-            float val = 0.f;
-            if (fi < total) {
-                const int e = e0 + fi / n_vars, va = fi % n_vars;
-                const long long o = (long long)loc_site[e] * n_vars + va;
-                if (k < M) val = dy[o * M + k];
-                if (k == 0) {
-                    sW[r] = loc_w[e] * coef[va];
-                    sE[r] = dyo[o];
+    // GRAM_RUN gridpoints of a workgroup; most analyses leave none
+    const int run0 = blockIdx.x * GRAM_RUN, lane = t & 63;
+    unsigned long long todo = __ballot(lane < GRAM_RUN && run0 + lane < nodes && left[run0 + lane]);
+    for (; todo; todo &= todo - 1) {
+        const int g = run0 + __builtin_ctzll(todo);
+        float acc[4][4] = {};
+        float bacc[4] = {};
+        const int e0 = loc_ptr[g], e1 = loc_ptr[g + 1];
+        const int total = (e1 - e0) * n_vars;
+        for (int base = 0; base < total; base += GRAM_CH) {
+            for (int idx = t; idx < GRAM_CH * GRAM_MP; idx += GRAM_NT) {
+                const int r = idx / GRAM_MP, k = idx % GRAM_MP;
+                const int fi = base + r;
+                float val = 0.f;
+                if (fi < total) {
+                    const int e = e0 + fi / n_vars, va = fi % n_vars;
+                    const long long o = (long long)loc_site[e] * n_vars + va;
+                    if (k < M) val = dy[o * M + k];
+                    if (k == 0) {
+                        sW[r] = loc_w[e] * coef[va];
+                        sE[r] = dyo[o];
+                    }
+                } else if (k == 0) {
+                    sW[r] = 0.f;
+                    sE[r] = 0.f;
                 }
-            } else if (k == 0) {
-                sW[r] = 0.f;
-                sE[r] = 0.f;
+                sD[r][k] = val;
             }
-            sD[r][k] = val;
-        }
-        __syncthreads();
-        if (active) {
-            for (int r = 0; r < GRAM_CH; ++r) {
-                const float w = sW[r];
-                float a[4], bb[4];
+            __syncthreads();
+            if (active) {
+                for (int r = 0; r < GRAM_CH; ++r) {
+                    const float w = sW[r];
+                    float a[4], bb[4];
 #pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    a[x] = sD[r][4 * kb + x];
-                    bb[x] = sD[r][4 * lb + x];
-                }
+                    for (int x = 0; x < 4; ++x) {
+                        a[x] = sD[r][4 * kb + x];
+                        bb[x] = sD[r][4 * lb + x];
+                    }
 #pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    const float wa = w * a[x];
+                    for (int x = 0; x < 4; ++x) {
+                        const float wa = w * a[x];
 #pragma unroll
-                    for (int y = 0; y < 4; ++y) acc[x][y] += wa * bb[y];
-                }
-                if (lb == 0) {
-                    const float we = w * sE[r];
+                        for (int y = 0; y < 4; ++y) acc[x][y] += wa * bb[y];
+                    }
+                    if (lb == 0) {
+                        const float we = w * sE[r];
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) bacc[x] += we * a[x];
+                        for (int x = 0; x < 4; ++x) bacc[x] += we * a[x];
+                    }
                 }
             }
+            __syncthreads();
         }
-        __syncthreads();
+        if (!active) continue;
+        float* Cg = gram + (long long)g * M * M;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const int k = 4 * kb + x;
+            if (k >= M) continue;
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                const int l = 4 * lb + y;
+                if (l >= M) continue;
+                Cg[k * M + l] = acc[x][y] + (k == l ? diag : 0.f);
+            }
+            if (lb == 0) bvec[(long long)g * M + k] = bacc[x];
+        }
     }
-    if (!active) return;
-    float* Cg = gram + (long long)g * M * M;
+}
+
+// ----------------------------------------------------------------------------
+// The plain analysis by series in FP64 (letkf_series.hpp), one wavefront per gridpoint:
+// the same C = (M-1)/beta I + dY^T Rl^-1 dY in FP32, here on the FP32 matrix cores
+// (v_mfma_f32_16x16x4f32: FP32 products and sums), kept in the accumulators and widened
+// there; then the update by products on the FP64 matrix cores.  The FP32 accumulators
+// hold rows 4 g + r where the FP64 ones hold g + 4 r, so the columns of the FP32 product
+// are gathered in the order member(c) = 4 (c % 4) + c / 4: row and column j of the FP64
+// matrix are then both member(j).  left[g]: what the eigensolve still has to do (a local
+// problem of condition above 65500, or a dumped gridpoint).
+// Bound by the FP64 matrix cores: 96^2 x 64 takes 0.66 ms, against 1.34 ms for C and
+// 64.8 ms for the eigensolve in LDS.
+// ----------------------------------------------------------------------------
+struct SeriesParams {
+    int M, nodes, n_vars, dump_g0, dump_n;
+    long long member_stride;
+    float diag;
+    float coef[3];
+    double sqm1;
+};
+
+template <int N>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(N == 64 ? 1 : 2, N == 64 ? 1 : 4))) void
+k_series_fp64(const int* __restrict__ loc_ptr, const int* __restrict__ loc_site, const float* __restrict__ loc_w,
+              const float* __restrict__ dy, const float* __restrict__ dyo, float* __restrict__ f, SeriesParams p,
+              const double4* __restrict__ table, int* __restrict__ status, unsigned char* __restrict__ left) {
+    constexpr int NT = N / 16;
+    __shared__ __align__(16) f64x4 basis[4 * NT * 64];
+    const int nb = gridDim.x;  // a multiple of 8: each XCD takes a contiguous range
+    const int g = int(blockIdx.x % 8) * (nb / 8) + int(blockIdx.x / 8);
+    if (g >= p.nodes) return;
+    const int lane = threadIdx.x, c = lane & 15, grp = lane >> 4;
+    const int M = p.M, nv = p.n_vars;
+    if (g >= p.dump_g0 && g < p.dump_g0 + p.dump_n) {
+        if (lane == 0) left[g] = 1;
+        return;
+    }
+    // C and b: lane group grp takes one of four observations per product
+    f32x4 acc[NT * NT + NT];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-        const int k = 4 * kb + x;
-        if (k >= M) continue;
+    for (int t = 0; t < NT * NT + NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int e0 = loc_ptr[g], P = (loc_ptr[g + 1] - e0) * nv;
+    const int cp = 4 * (c % 4) + c / 4;
+    constexpr int ST = 4;  // products in flight
+    for (int base = 0; base < P; base += 4 * ST) {
+        float xr[ST][NT], xc[ST][NT], yo[ST], w[ST];
 #pragma unroll
-        for (int y = 0; y < 4; ++y) {
-            const int l = 4 * lb + y;
-            if (l >= M) continue;
-            Cg[k * M + l] = acc[x][y] + (k == l ? diag : 0.f);
+        for (int s = 0; s < ST; ++s) {
+            const int j = base + 4 * s + grp;
+            const bool ok = j < P;
+            const int e = e0 + (ok ? j / nv : 0), va = ok ? j % nv : 0;
+            const int o = loc_site[e] * nv + va;
+            w[s] = ok ? loc_w[e] * (va == 0 ? p.coef[0] : (va == 1 ? p.coef[1] : p.coef[2])) : 0.f;
+#pragma unroll
+            for (int I = 0; I < NT; ++I) {
+                const int mr = 16 * I + c, mc = 16 * I + cp;
+                xr[s][I] = dy[(long long)o * M + (mr < M ? mr : 0)];
+                xc[s][I] = dy[(long long)o * M + (mc < M ? mc : 0)];
+                xr[s][I] = mr < M ? xr[s][I] : 0.f;
+                xc[s][I] = mc < M ? xc[s][I] : 0.f;
+            }
+            yo[s] = dyo[o];
         }
-        if (lb == 0) bvec[(long long)g * M + k] = bacc[x];
+#pragma unroll
+        for (int s = 0; s < ST; ++s)
+#pragma unroll
+            for (int I = 0; I < NT; ++I) {
+                const float wa = w[s] * xr[s][I];
+#pragma unroll
+                for (int J = 0; J < NT; ++J)
+                    acc[I * NT + J] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa, xc[s][J], acc[I * NT + J], 0, 0, 0);
+                acc[NT * NT + I] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa, c == 9 ? yo[s] : 0.f, acc[NT * NT + I], 0, 0, 0);
+            }
+    }
+    float trace = 0.f;
+#pragma unroll
+    for (int I = 0; I < NT; ++I)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) trace += 4 * grp + k == cp ? acc[I * NT + I][k] : 0.f;
+    if (__any(trace != trace)) {
+        // a NaN in the observed ensemble: every analysed value is NaN, whatever the solver
+        if (lane == 0) left[g] = 0;
+        if (c < Q) {
+            for (int l = grp; l < M; l += 4) f[(long long)l * p.member_stride + (long long)c * p.nodes + g] = quiet_nan();
+            atomicOr(status, 1);
+        }
+        return;
+    }
+    SeriesMat64<N> m;
+#pragma unroll
+    for (int t = 0; t < NT * NT; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m.t[t][k] = double(acc[t][k]);
+    // variable c of members 16 T + 4 grp + k; b in column 9
+    const float* fq = f + (long long)(c < Q ? c : 0) * p.nodes + g;
+    f64x4 r[NT];
+    double sum = 0;
+#pragma unroll
+    for (int T = 0; T < NT; ++T)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int l = 16 * T + 4 * grp + k;
+            r[T][k] = double(fq[(long long)(l < M ? l : 0) * p.member_stride]);
+            sum += l < M ? r[T][k] : 0.0;
+        }
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    const double xbar = sum / double(M);
+#pragma unroll
+    for (int T = 0; T < NT; ++T)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double dx = c < Q && 16 * T + 4 * grp + k < M ? r[T][k] - xbar : 0.0;
+            r[T][k] = c == 9 ? double(acc[NT * NT + T][k]) : dx;
+        }
+    const int steps = series_apply64<N>(m, r, double(p.diag), table, basis, lane);
+    if (lane == 0) left[g] = steps == 0;
+    if (steps == 0) return;
+    double dw = 0;  // dX w, w = C^-1 b in column 9
+#pragma unroll
+    for (int T = 0; T < NT; ++T) {
+        const f64x4 dx = basis[T * 64 + lane];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) dw = fma(dx[k], __shfl(r[T][k], (lane & 48) | 9), dw);
+    }
+    dw += __shfl_xor(dw, 16);
+    dw += __shfl_xor(dw, 32);
+    if (c < Q) {
+        float* fo = f + (long long)c * p.nodes + g;
+        bool bad = false;
+#pragma unroll
+        for (int T = 0; T < NT; ++T)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int l = 16 * T + 4 * grp + k;
+                if (l >= M) continue;
+                const float xa = float(xbar + fma(p.sqm1, r[T][k], dw));
+                bad |= !isfinite(xa);
+                fo[(long long)l * p.member_stride] = xa;
+            }
+        if (bad) atomicOr(status, 1);
     }
 }
 
@@ -310,8 +459,9 @@ template <int N>
 __global__ __launch_bounds__(64) void k_solve_fp64(const float* __restrict__ gram,
                                                    const float* __restrict__ bvec,
                                                    float* __restrict__ f, SolveParams sp,
-                                                   double* __restrict__ dump,
-                                                   int* __restrict__ status) {
+                                                   double* __restrict__ dump, int* __restrict__ status,
+                                                   const unsigned char* __restrict__ left) {
+    if (!left[blockIdx.x]) return;
     constexpr int NP = N / 2;
     constexpr int LD = N + 1;
     __shared__ double A[N * LD];
@@ -542,17 +692,48 @@ hipError_t launch_observe(Ctx& c, const double* hx_member, float* yo, uint64_t s
 }
 
 hipError_t launch_gram_fp32(Ctx& c) {
-    if (!c.d_gram || !c.d_bvec || !c.d_loc_ptr || !c.d_dy || !c.d_dyo) return hipErrorInvalidValue;
+    if (!c.d_gram || !c.d_bvec || !c.d_loc_ptr || !c.d_dy || !c.d_dyo || !c.d_left) return hipErrorInvalidValue;
     const float diag = float(double(c.M - 1) / c.cfg.inflation);
-    k_gram_fp32<<<int(c.nodes), GRAM_NT, 0, c.stream>>>(c.d_loc_ptr, c.d_loc_site, c.d_loc_w,
+    k_gram_fp32<<<int((c.nodes + GRAM_RUN - 1) / GRAM_RUN), GRAM_NT, 0, c.stream>>>(c.d_loc_ptr, c.d_loc_site, c.d_loc_w,
                                                         c.d_dy, c.d_dyo, c.d_obs_coef,
                                                         c.obs.n_vars, c.M, diag, c.d_gram,
-                                                        c.d_bvec);
+                                                        c.d_bvec, c.d_left, int(c.nodes));
+    return hipGetLastError();
+}
+
+const std::vector<double>& series_table64() {
+    static const std::vector<double> t = series_table<double>(SERIES_CLASSES64, SERIES_EPS64);
+    return t;
+}
+
+hipError_t launch_series_fp64(Ctx& c, float* f) {
+    if (!c.d_series64 || !c.d_left || !c.d_loc_ptr || !c.d_dy || !c.d_dyo || !f) return hipErrorInvalidValue;
+    SeriesParams p{};
+    p.M = c.M;
+    p.nodes = int(c.nodes);
+    p.n_vars = c.obs.n_vars;
+    p.dump_g0 = c.dump_g0;
+    p.dump_n = c.dump_n;
+    p.member_stride = c.lp.member_stride;
+    p.diag = float(double(c.M - 1) / c.cfg.inflation);
+    for (int a = 0; a < 3; ++a) p.coef[a] = c.obs.inv_sigma2[a];
+    p.sqm1 = sqrt(double(c.M - 1));
+    const dim3 grid(unsigned((c.nodes + 7) / 8 * 8));
+#define SERIES64(NN)                                                                                          \
+    k_series_fp64<NN><<<grid, 64, 0, c.stream>>>(c.d_loc_ptr, c.d_loc_site, c.d_loc_w, c.d_dy, c.d_dyo, f, p, \
+                                                 c.d_series64, c.d_status, c.d_left)
+    if (c.M <= 16)
+        SERIES64(16);
+    else if (c.M <= 32)
+        SERIES64(32);
+    else
+        SERIES64(64);
+#undef SERIES64
     return hipGetLastError();
 }
 
 hipError_t launch_solve_fp64(Ctx& c, float* f, unsigned long long* sweeps) {
-    if (!c.d_gram || !c.d_bvec || !f || (c.dump_n > 0 && !c.d_dump)) return hipErrorInvalidValue;
+    if (!c.d_gram || !c.d_bvec || !f || !c.d_left || (c.dump_n > 0 && !c.d_dump)) return hipErrorInvalidValue;
     SolveParams sp;
     sp.sweeps = sweeps;
     sp.M = c.M;
@@ -566,12 +747,12 @@ hipError_t launch_solve_fp64(Ctx& c, float* f, unsigned long long* sweeps) {
     while (N < c.M) N *= 2;
     const dim3 grid(unsigned(c.nodes)), block(64);
     switch (N) {
-        case 2: k_solve_fp64<2><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status); break;
-        case 4: k_solve_fp64<4><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status); break;
-        case 8: k_solve_fp64<8><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status); break;
-        case 16: k_solve_fp64<16><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status); break;
-        case 32: k_solve_fp64<32><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status); break;
-        case 64: k_solve_fp64<64><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status); break;
+        case 2: k_solve_fp64<2><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status, c.d_left); break;
+        case 4: k_solve_fp64<4><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status, c.d_left); break;
+        case 8: k_solve_fp64<8><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status, c.d_left); break;
+        case 16: k_solve_fp64<16><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status, c.d_left); break;
+        case 32: k_solve_fp64<32><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status, c.d_left); break;
+        case 64: k_solve_fp64<64><<<grid, block, 0, c.stream>>>(c.d_gram, c.d_bvec, f, sp, c.d_dump, c.d_status, c.d_left); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -41,8 +41,6 @@
 //
 // The workspace round trip (4 N^2 bytes per gridpoint each way) costs ~0.3 ms at
 // 256^2 x 64 and lets each kernel have the register budget of its own phase.
-#include <cstring>
-
 #include "context.hpp"
 #include "letkf_series.hpp"
 
@@ -1144,6 +1142,20 @@ __device__ __forceinline__ void series_body(int bx, int nbx, const int* __restri
     int ln = lane;
     asm volatile("" : "+v"(ln));  // addresses formed here, not held through the Gram matrix
     const int c = ln & 15, grp = ln >> 4;
+    float trace = 0.f;
+#pragma unroll
+    for (int I = 0; I < NT; ++I)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) trace += 4 * grp + k == c ? acc[I * NT + I][k] : 0.f;
+    if (__any(trace != trace)) {
+        // a NaN in the observed ensemble: every analysed value is NaN, whatever the solver
+        if (lane == 0) left[g] = 0;
+        if (mp.write_state && c < Q) {
+            for (int l = grp; l < M; l += 4) f[(long long)l * mp.member_stride + (long long)c * mp.nodes + g] = quiet_nan();
+            atomicOr(status, 1);
+        }
+        return;
+    }
     const float* fq = f + (long long)(c < Q ? c : 0) * mp.nodes + g;
     f32x4 r[NT];
     double sum = 0.0;
@@ -1231,12 +1243,15 @@ __device__ __forceinline__ void analysis_body(int bx, int nbx, const int* __rest
     const int gx = blk % mp.nx;
     const int gy0 = (blk / mp.nx) * mp.chain;
     const int gy1 = min(gy0 + mp.chain, mp.ny);
+    // the rows of the chain (at most 64) that are left to do
+    const unsigned long long todo = __ballot(gy0 + lane < gy1 && left[(gy0 + lane) * mp.nx + gx]);
+    if (todo == 0) return;
     bool bad = false;
     int sweeps = 2;
     bool warm = false;  // the previous gridpoint of the chain left its eigenvectors in cv
     for (int gy = gy0; gy < gy1; ++gy) {
         const int g = gy * mp.nx + gx;
-        if (!left[g]) {
+        if (!(todo >> (gy - gy0) & 1)) {
             warm = false;
             continue;
         }
@@ -1789,8 +1804,10 @@ MixedParams mixed_params(const Ctx& c, unsigned long long* sweeps32, unsigned lo
 
 }  // namespace
 
-size_t series_table_bytes() { return series_table().size() * sizeof(float); }
-const float* series_table_host() { return series_table().data(); }
+const std::vector<float>& series_table32() {
+    static const std::vector<float> t = series_table<float>(SERIES_CLASSES32, SERIES_EPS32);
+    return t;
+}
 
 int mixed_width(int M) {
     int N = 16;

@@ -22,8 +22,8 @@
 // matrix is the B operand of K-block K and, the matrix being symmetric, the tile (K, I)
 // its A operand.  No value moves between lanes from the Gram matrix to the analysed state.
 #pragma once
+#include <algorithm>
 #include <cmath>
-#include <mutex>
 #include <vector>
 
 #include "context.hpp"
@@ -31,60 +31,64 @@
 namespace lbmletkf {
 
 // ---- the series, on the host ------------------------------------------------------
-// Classes of condition number kappa = 2^(k/4), k = 1..SERIES_CLASSES; per class the
-// degree that leaves the series of x^(-1/2) and 1/x on [1, kappa] off by about 3e-8 of
-// their value at 1, and the coefficients d_kj of both.
-constexpr int SERIES_CLASSES = 40;    // kappa up to 1024
-constexpr int SERIES_CLASS0 = 64;     // float4 entries of the header (first entry of each class)
+// Classes of condition number kappa = 2^(k/4), k = 1, 2, ..; per class the degree that
+// leaves the series of x^(-1/2) and 1/x on [1, kappa] off by about eps of their value at
+// 1, and the coefficients d_kj of both.
+constexpr int SERIES_CLASS0 = 80;     // quadruples of the header (first quadruple of each class)
+// The widest class lies where the eigensolve of the same kernel family costs as much: in
+// the mixed analysis at N = 64 a block product costs 1/110 of the warm-started sweeps
+// (kappa 2000), in FP64 1/4000 of them; there the table ends it (0.7 MB).
+constexpr int SERIES_CLASSES32 = 40, SERIES_CLASSES64 = 64;  // kappa up to 1024 and 65536
+constexpr double SERIES_EPS32 = 3e-8, SERIES_EPS64 = 1e-13;
 
-// table[class] = (first entry, blocks K, 0, 0) as ints in the header; then per block k
-// the two entries d_k0..d_k3 of x^(-1/2) and of 1/x
-inline const std::vector<float>& series_table() {
-    static std::vector<float> t;
-    static std::once_flag once;
-    std::call_once(once, [] {
-        std::vector<float> body;
-        t.assign(4 * SERIES_CLASS0, 0.f);
-        const double pi = 3.14159265358979323846;
-        for (int cl = 1; cl <= SERIES_CLASSES; ++cl) {
-            const double kappa = std::exp2(cl / 4.0);
-            int n = int(std::ceil(std::log(1.0 / 3e-8) / (2.0 * std::atanh(1.0 / std::sqrt(kappa))))) + 1;
-            const int K = std::max(2, (n + 3) / 4);
-            n = 4 * K;
-            const int P = 2 * n;  // quadrature nodes: aliases start at coefficient 3 n
-            std::vector<double> c[2];
-            c[0].assign(n, 0.0);
-            c[1].assign(n, 0.0);
-            for (int p = 0; p < P; ++p) {
-                const double x = std::cos(pi * (p + 0.5) / P);
-                const double y = 0.5 * ((kappa - 1.0) * x + kappa + 1.0);
-                const double f0 = 1.0 / std::sqrt(y), f1 = 1.0 / y;
-                double t0 = 1.0, t1 = x;
-                for (int k = 0; k < n; ++k) {
-                    c[0][k] += f0 * t0;
-                    c[1][k] += f1 * t0;
-                    const double t2 = 2.0 * x * t1 - t0;
-                    t0 = t1;
-                    t1 = t2;
-                }
-            }
-            int head[4] = {int(SERIES_CLASS0 + body.size() / 4), K, 0, 0};
-            std::memcpy(&t[4 * cl], head, sizeof head);
-            std::vector<double> d(size_t(K) * 8);
-            for (int f = 0; f < 2; ++f) {
-                for (int k = 0; k < n; ++k) c[f][k] *= (k == 0 ? 1.0 : 2.0) / P;
-                // T_{4k+j} = 2 T_4k T_j - T_{4(k-1) + (4-j)}
-                for (int k = K - 1; k >= 0; --k)
-                    for (int j = 0; j < 4; ++j) {
-                        const double ck = c[f][4 * k + j];
-                        d[size_t(k) * 8 + 4 * f + j] = k > 0 && j > 0 ? 2.0 * ck : ck;
-                        if (k > 0 && j > 0) c[f][4 * (k - 1) + 4 - j] -= ck;
-                    }
-            }
-            for (double x : d) body.push_back(float(x));
+// Quadruples of T: entry k of the header is (first quadruple, blocks K, 0, 0) of class k,
+// as values; then per block the two quadruples d_k0..d_k3 of x^(-1/2) and of 1/x.
+template <class T>
+std::vector<T> series_table(int classes, double eps) {
+    std::vector<T> t(4 * SERIES_CLASS0, T(0));
+    for (int cl = 1; cl <= classes; ++cl) {
+        const double kappa = std::exp2(cl / 4.0), q = (std::sqrt(kappa) - 1.0) / (std::sqrt(kappa) + 1.0);
+        const int degree = int(std::ceil(std::log(1.0 / eps) / -std::log(q))) + 1;
+        const int K = std::max(2, (degree + 3) / 4), n = 4 * K;
+        std::vector<double> c[2];
+        // 1/y, y = ((kappa-1) x + kappa + 1)/2: c_k = (2 - [k = 0]) (-q)^k / sqrt(kappa)
+        c[1].resize(n);
+        for (int k = 0; k < n; ++k) c[1][k] = (k ? 2.0 : 1.0) * std::pow(-q, k) / std::sqrt(kappa);
+        // y^(-1/2) = f: 2 (x + al) f' + f = 0, al = (kappa+1)/(kappa-1), gives for the
+        // coefficients d_k of f'
+        //   (1 + 1/2k) d_{k-1} + 2 al d_k + (1 - 1/2k) d_{k+1} = 0,  c_k = (d_{k-1} - d_{k+1})/2k,
+        // of which they are the decaying solution: taken downwards from far above the
+        // degree, and scaled to f = 1 at y = 1 (x = -1) and f = kappa^(-1/2) at x = 1
+        const double al = (kappa + 1.0) / (kappa - 1.0);
+        const int top = 2 * n + 40;
+        std::vector<double> d(top + 2, 0.0);
+        d[top] = 1e-280;
+        for (int k = top; k >= 1; --k)
+            d[k - 1] = -(2.0 * al * d[k] + (1.0 - 0.5 / k) * d[k + 1]) / (1.0 + 0.5 / k);
+        c[0].resize(n);
+        double lo = 0.0, hi = 0.0;  // sum_{k>0} of the unscaled series at x = -1 and x = 1
+        for (int k = top; k >= 1; --k) {
+            const double ck = (d[k - 1] - d[k + 1]) / (2.0 * k);
+            lo += k % 2 ? -ck : ck;
+            hi += ck;
+            if (k < n) c[0][k] = ck;
         }
-        t.insert(t.end(), body.begin(), body.end());
-    });
+        const double scale = (1.0 - 1.0 / std::sqrt(kappa)) / (lo - hi);
+        for (int k = 1; k < n; ++k) c[0][k] *= scale;
+        c[0][0] = 1.0 - scale * lo;
+        t[4 * cl] = T(t.size() / 4);
+        t[4 * cl + 1] = T(K);
+        std::vector<double> e(size_t(K) * 8);
+        for (int f = 0; f < 2; ++f)
+            // T_{4k+j} = 2 T_4k T_j - T_{4(k-1) + (4-j)}
+            for (int k = K - 1; k >= 0; --k)
+                for (int j = 0; j < 4; ++j) {
+                    const double ck = c[f][4 * k + j];
+                    e[size_t(k) * 8 + 4 * f + j] = k > 0 && j > 0 ? 2.0 * ck : ck;
+                    if (k > 0 && j > 0) c[f][4 * (k - 1) + 4 - j] -= ck;
+                }
+        for (double x : e) t.push_back(T(x));
+    }
     return t;
 }
 
@@ -96,6 +100,8 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float quiet_nan() { return __int_as_float(0x7fc00000); }
 
 // Operands of one K-block: two accumulator tiles (32 values of k), or the only one of a
 // 16 x 16 problem.
@@ -267,13 +273,13 @@ __device__ __forceinline__ int series_apply(const f32x4* acc, f32x4 (&r)[N / 16]
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
     const float kappa = 1.f + 1.0001f * __builtin_amdgcn_sqrtf(__builtin_amdgcn_sqrtf(ss)) / a;
-    if (!(kappa <= 1023.f)) return 0;
+    if (!(kappa <= 1023.f)) return 0;  // SERIES_CLASSES32
     const int cl = __builtin_amdgcn_readfirstlane(max(1, int(ceilf(4.f * log2f(kappa)))));
     const float lam = a * (exp2f(0.25f * float(cl)) - 1.f);
     const float al = 2.f / lam;  // x = al A - 1
     const float4 hd = table[cl];
-    const int first = __builtin_amdgcn_readfirstlane(__float_as_int(hd.x));
-    const int K = __builtin_amdgcn_readfirstlane(__float_as_int(hd.y));
+    const int first = __builtin_amdgcn_readfirstlane(int(hd.x));
+    const int K = __builtin_amdgcn_readfirstlane(int(hd.y));
 
     // V_0 = r, V_1 = x V_0, V_j = 2 x V_{j-1} - V_{j-2}
     {
@@ -352,6 +358,148 @@ __device__ __forceinline__ int series_apply(const f32x4* acc, f32x4 (&r)[N / 16]
     }
     // f(C) = a^(-1/2) f(C / a), 1 / C = (1/a) 1 / (C / a)
     const float scale = c == 9 ? 1.f / a_in : 1.f / sqrtf(a_in);
+#pragma unroll
+    for (int T = 0; T < NT; ++T) r[T] = b1[T] * scale;
+    return K + 2;
+}
+
+// ---- the same in FP64 (the PLAIN variant), on v_mfma_f64_16x16x4f64 ------------------
+// A[m][k] from lane (m = lane % 16, k = lane / 16), B[k][n] from lane (n = lane % 16,
+// k = lane / 16), D[lane / 16 + 4 r][lane % 16]: summed over k in the order (T, r), the
+// accumulator tiles are operands as they stand here too.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+template <int N>
+struct SeriesMat64 {
+    static constexpr int NT = N / 16;
+    f64x4 t[NT * NT];  // tile (K, J)
+    __device__ __forceinline__ void square(f64x4 (&d)[NT * NT]) const {
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) d[i * NT + j] = f64x4{0, 0, 0, 0};
+#pragma unroll
+        for (int K = 0; K < NT; ++K)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        d[i * NT + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(t[K * NT + i][r], t[K * NT + j][r],
+                                                                             d[i * NT + j], 0, 0, 0);
+    }
+    // c += this * (s v)
+    __device__ __forceinline__ void times(const f64x4 (&v)[NT], double s, f64x4 (&c)[NT]) const {
+#pragma unroll
+        for (int K = 0; K < NT; ++K)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double x = s * v[K][r];
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+                    c[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(t[K * NT + i][r], x, c[i], 0, 0, 0);
+            }
+    }
+};
+
+// r := f(C) r, as series_apply; m holds A and is overwritten; basis: 4 N 16 doubles of
+// LDS, basis[(j NT + T) 64 + lane] the incoming r (j = 0) afterwards.
+template <int N>
+__device__ __forceinline__ int series_apply64(SeriesMat64<N>& m, f64x4 (&r)[N / 16], double a,
+                                              const double4* __restrict__ table, f64x4* basis, int lane) {
+    constexpr int NT = N / 16;
+    auto put = [&](int j, const f64x4 (&x)[NT]) {
+#pragma unroll
+        for (int T = 0; T < NT; ++T) basis[(j * NT + T) * 64 + lane] = x[T];
+    };
+    auto get = [&](int j, int T) { return basis[(j * NT + T) * 64 + lane]; };
+    const double ia = 1.0 / a;
+    f64x4 sq[NT * NT];
+#pragma unroll
+    for (int t = 0; t < NT * NT; ++t) m.t[t] *= ia;  // spectrum [0, kappa - 1]
+    m.square(sq);
+    double ss = 0;
+#pragma unroll
+    for (int t = 0; t < NT * NT; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) ss = fma(sq[t][k], sq[t][k], ss);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+    const float kappa = 1.f + 1.0001f * float(sqrt(sqrt(ss)));
+    if (!(kappa <= 65500.f)) return 0;  // SERIES_CLASSES64
+    const int cl = __builtin_amdgcn_readfirstlane(max(1, int(ceilf(4.f * log2f(kappa)))));
+    const double lam = exp2(0.25 * double(cl)) - 1.0;
+    const double al = 2.0 / lam;
+    const double4 hd = table[cl];
+    const int first = __builtin_amdgcn_readfirstlane(int(hd.x));
+    const int K = __builtin_amdgcn_readfirstlane(int(hd.y));
+    {
+        f64x4 v[NT];
+        put(0, r);
+#pragma unroll
+        for (int T = 0; T < NT; ++T) v[T] = -r[T];
+        m.times(r, al, v);
+        put(1, v);
+#pragma unroll
+        for (int j = 2; j < 4; ++j) {
+            f64x4 w[NT];
+#pragma unroll
+            for (int T = 0; T < NT; ++T) w[T] = -2.0 * v[T] - get(j - 2, T);
+            m.times(v, 2.0 * al, w);
+            put(j, w);
+#pragma unroll
+            for (int T = 0; T < NT; ++T) v[T] = w[T];
+        }
+    }
+    // T_2 = 2 al^2 A^2 - 4 al A + I; 2 T_4 = 4 T_2^2 - 2 I
+    const int c = lane & 15, g = lane >> 4;
+    const double k2 = 2.0 * al * al, k1 = -4.0 * al;
+#pragma unroll
+    for (int I = 0; I < NT; ++I)
+#pragma unroll
+        for (int J = 0; J < NT; ++J)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                m.t[I * NT + J][k] = fma(k2, sq[I * NT + J][k],
+                                         fma(k1, m.t[I * NT + J][k], I == J && g + 4 * k == c ? 1.0 : 0.0));
+    m.square(sq);
+#pragma unroll
+    for (int I = 0; I < NT; ++I)
+#pragma unroll
+        for (int J = 0; J < NT; ++J)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                m.t[I * NT + J][k] = fma(4.0, sq[I * NT + J][k], I == J && g + 4 * k == c ? -2.0 : 0.0);
+    const double4* coef = table + first + (c == 9 ? 1 : 0);
+    f64x4 b1[NT], b2[NT];
+    {
+        const double4 d = coef[2 * (K - 1)];
+#pragma unroll
+        for (int T = 0; T < NT; ++T) {
+            b1[T] = d.x * get(0, T) + d.y * get(1, T) + d.z * get(2, T) + d.w * get(3, T);
+            b2[T] = f64x4{0, 0, 0, 0};
+        }
+    }
+#pragma unroll 1
+    for (int k = K - 2; k >= 0; --k) {
+        const double4 d = coef[2 * k];
+        f64x4 q[NT];
+#pragma unroll
+        for (int T = 0; T < NT; ++T) {
+            const f64x4 x0 = get(0, T), x1 = get(1, T), x2 = get(2, T), x3 = get(3, T);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                q[T][e] = fma(d.x, x0[e], fma(d.y, x1[e], fma(d.z, x2[e], fma(d.w, x3[e], -b2[T][e]))));
+        }
+        m.times(b1, k > 0 ? 1.0 : 0.5, q);
+#pragma unroll
+        for (int T = 0; T < NT; ++T) {
+            b2[T] = b1[T];
+            b1[T] = q[T];
+        }
+    }
+    const double scale = c == 9 ? ia : sqrt(ia);
 #pragma unroll
     for (int T = 0; T < NT; ++T) r[T] = b1[T] * scale;
     return K + 2;
