@@ -1090,15 +1090,16 @@ struct LbmShape {
 };
 
 // Time of one strip launch, in arbitrary units: a strip of r rows walks r + halo row
-// iterations, each taking 3 + 2 w with w wavefronts on a SIMD (256^2, three steps: 1.25,
-// 1.85 and 2.75 us at w = 1, 2, 4), in as many generations as the grid needs.
+// iterations, each taking 3 + 1.25 w with w wavefronts on a SIMD (three steps: 1.3 us at
+// w = 1, 1.6 at 1.7 and 2, 1.9 at 2.6, 2.1 to 2.7 at 4), in as many generations as the
+// grid needs.
 static double strip_cost(const Ctx& c, int r, int halo, size_t lds_per_column) {
     const int waves = (c.nx + 63) / 64;
     const long long wgs = (long long)((c.ny + r - 1) / r) * c.M;
     const long long per_cu = std::min<long long>((160 * 1024) / (long long)(lds_per_column * c.nx), 16 / waves);
     const long long slots = 256 * std::max(1LL, per_cu);
-    const double w = std::ceil(double(std::min(wgs, slots)) * waves / 1024.0);
-    return (r + halo) * (3.0 + 2.0 * w) * std::max(1.0, double(wgs) / double(slots));
+    const double w = std::max(1.0, double(std::min(wgs, slots)) * waves / 1024.0);
+    return (r + halo) * (3.0 + 1.25 * w) * std::max(1.0, double(wgs) / double(slots));
 }
 
 // The shape of a context whose shape was not set.  Measured us per step (256 CUs):
@@ -1124,7 +1125,7 @@ static LbmShape default_shape(const Ctx& c) {
     const bool three = c.nx <= 512;
     LbmShape best = blocks;
     double cost = 0;
-    for (int r : {4, 6, 8, 12, 16, 24, 32}) {
+    for (int r : {4, 6, 8, 16, 24, 32}) {
         const double t = three ? strip_cost(c, r, 10, 36 * 4) : strip_cost(c, r, 6, (12 + 3 * P1Q) * 4);
         if (best.rows == 0 || t < cost) {
             best = {three ? 3 : 2, r, 0};
