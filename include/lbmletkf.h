@@ -93,7 +93,7 @@ typedef struct lbmletkf_config {
     int    variant;             /* LBMLETKF_VARIANT_*                                       */
     double jacobi_tol;          /* relative off-diagonal tolerance of the eigensolver (where one is taken: a local problem of condition above 65500 (PLAIN) or 1023 (MIXED), a dumped gridpoint) */
     int    jacobi_max_sweeps;   /* cusolver syevj uses tol 1e-6, 100 sweeps (cu_matrix_eigensolver_wrapper.hpp:192-193) */
-    int    gram_passes;         /* MIXED: 1 = bf16 operands, 3 = split bf16 (hi*hi + hi*lo + lo*hi) */
+    int    gram_passes;         /* MIXED: 1 = 16-bit operands, 3 = split in two (hi*hi + hi*lo + lo*hi) */
     int    jacobi_fp64_sweeps;  /* MIXED: at most this many FP64 sweeps after the FP32 phase (presets: 0) */
     /* eddy-viscosity closure of the fused LBM kernel (MIXED variant) */
     int    closure_kind;         /* LBMLETKF_CLOSURE_*                                       */

@@ -7,7 +7,7 @@
 // k_mixed_analysis: gather, Gram matrix, FP32 Jacobi sweeps and update of the
 //     gridpoints the series left (condition number above 1023, or dumped: the dump
 //     records eigenpairs).
-// At 256^2 x 64 (kappa ~ 20) the first takes 1.2 ms and the second, with nothing left
+// At 256^2 x 64 (kappa ~ 20) the first takes 0.64 ms and the second, with nothing left
 // to do, 9 us; the sweeps take 5.1 ms for the same gridpoints.
 //
 // With FP64 sweeps, two kernels:
@@ -48,6 +48,9 @@ namespace lbmletkf {
 
 namespace {
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
 struct MixedParams {
     int M, nodes, n_vars;
     int n_obs;              // scalar observations (rows of dY)
@@ -65,7 +68,8 @@ struct MixedParams {
     int chain;              // k_mixed_solve: consecutive gridpoints per wavefront
     int write_state;        // k_mixed_analysis: 0 skips the state update (timing only)
     const float4* series;   // k_series_analysis: coefficients of the series (letkf_series.hpp)
-    float series_scale;     // the power of two that brings diag to [1, 2)
+    float gram_scale;       // k_series_analysis: the power of two applied to the rows of dY
+    float gram_scale2;      // its square, which brings diag to [16, 64)
     unsigned long long* series_steps;  // block products summed over gridpoints (may be null)
     unsigned long long* sweeps32;
     unsigned long long* sweeps64;
@@ -1112,21 +1116,186 @@ __device__ inline void warm_start_acc(const f32x4 (&acc)[GRAM_FULL<N>], float* c
 // ---------------------------------------------------------------------------------
 // The analysis by series (letkf_series.hpp), one wavefront per gridpoint, nothing
 // carried from one gridpoint to the next: gather and Gram matrix as above, then lane
-// (c, grp) takes variable c of members 16 T + 4 grp + r (c < 9), column 9 of the block
+// (c, grp) takes variable c of members NT (4 grp + r) + T (c < 9), column 9 of the block
 // is b.  left[g] tells the kernel of the sweeps what it still has to do: the gridpoints
 // whose local problem is too badly conditioned for the series, and those dumped.
+// Bound by instruction issue: at 256^2 x 64 about 3200 vector instructions of 4 cycles and
+// 512 of the matrix cores of 16 per gridpoint, which add up to the kernel's time at three
+// wavefronts per SIMD (0.64 ms; 0.70 at 11 wavefronts per CU, where 1 KB more of LDS ends).
+// With three bf16 parts, all tiles computed and two wavefronts per SIMD it took 1.19 ms.
 // ---------------------------------------------------------------------------------
 template <int N>
 struct SeriesShared {
-    float basis[N == 64 ? 4 * 64 * 16 : 4];
+    float basis[N == 64 ? 11 * 64 * 4 : 4];
+    float mirror[N > 16 ? MIRROR_TILE : 4];
 };
+static_assert((sizeof(SeriesShared<64>) + 1279) / 1280 * 12 <= 128, "three wavefronts per SIMD");
+
+// Rows of dY (times sqrt(R^-1 o localization)) of the local observations in f16 hi + lo
+// parts, their Gram matrix in acc (tiles I NT + J with I <= J, scaled by gram_scale^2), and
+// b = G^T sqrt(R^-1) dyo, unscaled, in b[T] (FP32).  Row or column 16 T + c of the matrix is
+// member NT c + T, so that a lane loads its elements of a row of dY at once.  The order of the observations is free, so a lane takes, for chunks of 32 entries of the
+// local list, entries 4 t + lane / 16: one address and one weight for all variables of a
+// site, the (t, variable) pairs dealt to the K-blocks at compile time, and a last chunk's
+// empty K-blocks left out.  gram_scale brings sqrt((M-1)/beta) to [4, 8): f16 then resolves
+// rows to 2^-27 of it however small they are, rows that the series can take (G^T G at most
+// 1022 (M-1)/beta) stay in the range of f16, and what larger ones overflow to (not finite)
+// goes to the sweeps.
+// Per K-block at N = 64: about 160 vector instructions and 30 of the matrix cores, a third
+// of the kernel; bf16 parts with a division per observation took 436 and 60.
+__device__ __forceinline__ int row_ror8(int v) { return __builtin_amdgcn_mov_dpp(v, DPP_XOR8, 0xF, 0xF, true); }
+// the value of lane t of the row of 16 (t a constant after unrolling)
+__device__ __forceinline__ int row_bcast(int t, int v) {
+    switch (t) {
+#define LML_BCAST(T) case T: return __builtin_amdgcn_mov_dpp(v, 0x150 + T, 0xF, 0xF, true);
+        LML_BCAST(0) LML_BCAST(1) LML_BCAST(2) LML_BCAST(3) LML_BCAST(4) LML_BCAST(5) LML_BCAST(6)
+#undef LML_BCAST
+        default: return __builtin_amdgcn_mov_dpp(v, 0x157, 0xF, 0xF, true);
+    }
+}
+template <int N, int PASSES, int NV>
+__device__ __forceinline__ void series_gram_nv(int e0, int e1, int lane, const int* __restrict__ loc_site,
+                                               const float* __restrict__ loc_w, const float* __restrict__ dy,
+                                               const float* __restrict__ dyo, const MixedParams& mp,
+                                               f32x4 (&acc)[N / 16 * N / 16], float (&b)[N / 16]) {
+    constexpr int NT = N / 16;
+    const int M = mp.M;
+    const int col = lane & 15, kq = lane >> 4;
+    const __amdgpu_buffer_rsrc_t rdy =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(dy), 0, mp.n_obs * M * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rdyo =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(dyo), 0, mp.n_obs * 4, 0x00020000);
+    float cf[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+        cf[v] = __int_as_float(__builtin_amdgcn_readfirstlane(
+            __float_as_int(__builtin_amdgcn_sqrtf(mp.coef[v]) * mp.gram_scale)));
+    const int E = e1 - e0;
+    const __amdgpu_buffer_rsrc_t rsite =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(loc_site + e0), 0, E * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(loc_w + e0), 0, E * 4, 0x00020000);
+    const unsigned row = NV * M * 4;
+    int at, ao;  // byte offsets of the entry's rows of dY and of its innovations
+    float sw;
+    // entry base + 4 j + kq in lane (j, kq); past the end the last one, its weight read as 0
+    auto entry = [&](int base, unsigned& site, float& w) __attribute__((always_inline)) {
+        const int e4 = (base + 4 * col + kq) * 4;
+        site = __builtin_amdgcn_raw_buffer_load_b32(rsite, min(e4, E * 4 - 4), 0, 0);
+        w = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, e4, 0, 0));
+    };
+    unsigned site;
+    float w;
+    entry(0, site, w);
+    for (int b32 = 0; b32 < E; b32 += 32) {
+        if (b32 % 64 == 0) {
+            // 24-bit product where dY, below 2^31 bytes, has rows of more than 2^7
+            at = int(N > 32 ? __umul24(site, row) : site * row);
+            ao = site * (NV * 4);
+            sw = __builtin_amdgcn_sqrtf(w);
+            entry(b32 + 64, site, w);
+        } else {
+            at = row_ror8(at);
+            ao = row_ror8(ao);
+            sw = __int_as_float(row_ror8(__float_as_int(sw)));
+        }
+#pragma unroll
+        for (int s = 0; s < NV; ++s) {
+            if (s > 0 && b32 + 4 * (8 * s / NV) >= E) break;
+            float x[NT][8], y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int t = (8 * s + i) / NV, v = (8 * s + i) % NV;
+                const int vo = row_bcast(t, at) + (col * (4 * NT) + v * M * 4);
+                if constexpr (NT == 4) {
+                    const f32x4 q = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rdy, vo, 0, 0));
+#pragma unroll
+                    for (int I = 0; I < NT; ++I) x[I][i] = q[I];
+                } else if constexpr (NT == 2) {
+                    const f32x2 q = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rdy, vo, 0, 0));
+                    x[0][i] = q[0];
+                    x[1][i] = q[1];
+                } else {
+                    x[0][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rdy, vo, 0, 0));
+                }
+                if constexpr (NV == 2) {
+                    if (v == 0) {
+                        const f32x2 q = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rdyo, row_bcast(t, ao), 0, 0));
+                        y[i] = q[0];
+                        y[i + 1] = q[1];
+                    }
+                } else {
+                    y[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rdyo, row_bcast(t, ao) + 4 * v, 0, 0));
+                }
+            }
+            f16x8 p[NT][2];
+            float ws[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                ws[i] = __int_as_float(row_bcast((8 * s + i) / NV, __float_as_int(sw))) * cf[(8 * s + i) % NV];
+                y[i] *= ws[i];
+            }
+#pragma unroll
+            for (int I = 0; I < NT; ++I) {
+                f32x4 xs[2];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    xs[i / 4][i % 4] = x[I][i] * ws[i];
+                    b[I] = fmaf(xs[i / 4][i % 4], y[i], b[I]);
+                }
+                split_tiles(xs, p[I]);
+            }
+#pragma unroll
+            for (int q = PASSES == 3 ? 0 : 2; q < 3; ++q)
+#pragma unroll
+                for (int I = 0; I < NT; ++I)
+#pragma unroll
+                    for (int J = I; J < NT; ++J) acc[I * NT + J] = series_fma(q, p[I], p[J], acc[I * NT + J]);
+        }
+    }
+}
+template <int N, int PASSES>
+__device__ __forceinline__ void series_gram(int g, int lane, const int* __restrict__ loc_ptr,
+                                            const int* __restrict__ loc_site, const float* __restrict__ loc_w,
+                                            const float* __restrict__ dy, const float* __restrict__ dyo,
+                                            const MixedParams& mp, f32x4 (&acc)[N / 16 * N / 16],
+                                            float (&b)[N / 16]) {
+    constexpr int NT = N / 16;
+#pragma unroll
+    for (int i = 0; i < NT * NT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int T = 0; T < NT; ++T) b[T] = 0.f;
+    const int e0 = loc_ptr[g], e1 = loc_ptr[g + 1];
+    if (mp.n_vars == 1)
+        series_gram_nv<N, PASSES, 1>(e0, e1, lane, loc_site, loc_w, dy, dyo, mp, acc, b);
+    else if (mp.n_vars == 2)
+        series_gram_nv<N, PASSES, 2>(e0, e1, lane, loc_site, loc_w, dy, dyo, mp, acc, b);
+    else
+        series_gram_nv<N, PASSES, 3>(e0, e1, lane, loc_site, loc_w, dy, dyo, mp, acc, b);
+    const int c = lane & 15, grp = lane >> 4, M = mp.M;
+#pragma unroll
+    for (int T = 0; T < NT; ++T) {
+        b[T] += __shfl_xor(b[T], 16);
+        b[T] += __shfl_xor(b[T], 32);
+        b[T] = NT * c + T < M ? b[T] * pow2_inverse(mp.gram_scale2) : 0.f;
+    }
+    if (M < N) {  // tile elements of members >= M hold what follows their row
+#pragma unroll
+        for (int I = 0; I < NT; ++I)
+#pragma unroll
+            for (int J = I; J < NT; ++J)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (NT * (4 * grp + r) + I >= M || NT * c + J >= M) acc[I * NT + J][r] = 0.f;
+    }
+}
 
 template <int N, int PASSES>
 __device__ __forceinline__ void series_body(int bx, int nbx, const int* __restrict__ loc_ptr,
                                             const int* __restrict__ loc_site, const float* __restrict__ loc_w,
                                             const float* __restrict__ dy, const float* __restrict__ dyo,
                                             float* __restrict__ f, const MixedParams& mp, int* __restrict__ status,
-                                            unsigned char* __restrict__ left, float* lds) {
+                                            unsigned char* __restrict__ left, SeriesShared<N>& sh) {
     constexpr int NT = N / 16;
     const int lane = threadIdx.x;
     const int g = xcd_order(bx, nbx);
@@ -1137,8 +1306,9 @@ __device__ __forceinline__ void series_body(int bx, int nbx, const int* __restri
         if (lane == 0) left[g] = 1;
         return;
     }
-    f32x4 acc[GRAM_FULL<N>];
-    gram_acc<N, PASSES, true>(g, lane, loc_ptr, loc_site, loc_w, dy, dyo, mp, acc);
+    f32x4 acc[NT * NT];
+    float b[NT];
+    series_gram<N, PASSES>(g, lane, loc_ptr, loc_site, loc_w, dy, dyo, mp, acc, b);
     int ln = lane;
     asm volatile("" : "+v"(ln));  // addresses formed here, not held through the Gram matrix
     const int c = ln & 15, grp = ln >> 4;
@@ -1147,39 +1317,60 @@ __device__ __forceinline__ void series_body(int bx, int nbx, const int* __restri
     for (int I = 0; I < NT; ++I)
 #pragma unroll
         for (int k = 0; k < 4; ++k) trace += 4 * grp + k == c ? acc[I * NT + I][k] : 0.f;
-    if (__any(trace != trace)) {
-        // a NaN in the observed ensemble: every analysed value is NaN, whatever the solver
-        if (lane == 0) left[g] = 0;
-        if (mp.write_state && c < Q) {
+    if (__any(!isfinite(trace))) {
+        // past the range of f16, or of FP32 squares (a NaN in the observed ensemble): in
+        // the latter case every analysed value is NaN, whatever the solver
+        bool nan = false;
+        for (int e = loc_ptr[g]; e < loc_ptr[g + 1]; ++e)
+            for (int v = 0; v < mp.n_vars; ++v) {
+                const float x = dy[((long long)loc_site[e] * mp.n_vars + v) * M + (lane < M ? lane : 0)];
+                nan |= !(fabsf(x) * sqrtf(loc_w[e] * mp.coef[v]) < 1e18f);
+            }
+        nan = __any(nan);
+        if (lane == 0) left[g] = !nan;
+        if (nan && mp.write_state && c < Q) {
             for (int l = grp; l < M; l += 4) f[(long long)l * mp.member_stride + (long long)c * mp.nodes + g] = quiet_nan();
             atomicOr(status, 1);
         }
         return;
     }
+    // member NT (4 grp + k) + T: an address per lane and an offset per (T, k); past the last
+    // member the first one's address, whose value is not used.  Columns 10 to 15 repeat
+    // variable 0.
     const float* fq = f + (long long)(c < Q ? c : 0) * mp.nodes + g;
+    const float* fg = fq + 4 * NT * grp * mp.member_stride;
     f32x4 r[NT];
-    double sum = 0.0;
+    double xbar;
+    // (two copies of this: with as many members as rows nothing is masked)
+    auto perturbations = [&](auto ragged) __attribute__((always_inline)) {
+        double sum = 0.0;
 #pragma unroll
-    for (int T = 0; T < NT; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int l = 16 * T + 4 * grp + k;
-            r[T][k] = fq[(long long)(l < M ? l : 0) * mp.member_stride];
-            sum += l < M ? double(r[T][k]) : 0.0;
-        }
-    sum += __shfl_xor(sum, 16);
-    sum += __shfl_xor(sum, 32);
-    const double xbar = sum / double(M);
+            for (int k = 0; k < 4; ++k) {
+                const bool in = !ragged || NT * (4 * grp + k) + T < M;
+                r[T][k] = *(in ? fg + (NT * k + T) * mp.member_stride : fq);
+                sum += in ? double(r[T][k]) : 0.0;
+            }
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        xbar = sum / double(M);
 #pragma unroll
-    for (int T = 0; T < NT; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const bool in = 16 * T + 4 * grp + k < M;
-            const float dx = c < Q && in ? float(double(r[T][k]) - xbar) : 0.f;
-            r[T][k] = c == 9 ? acc[NT * NT + T][k] : dx;
-        }
-    SeriesBasis<N> basis(lds, lane);
-    const int steps = series_apply<N>(acc, r, mp.diag, mp.series_scale, mp.series, basis, lane);
+            for (int k = 0; k < 4; ++k) {
+                const bool in = !ragged || NT * (4 * grp + k) + T < M;
+                const float bl = __shfl(b[T], 4 * grp + k);
+                r[T][k] = c == 9 ? bl : in ? float(double(r[T][k]) - xbar) : 0.f;
+            }
+    };
+    if (M == N)
+        perturbations(std::false_type{});
+    else
+        perturbations(std::true_type{});
+    SeriesBasis<N> basis(sh.basis, lane);
+    float r0;
+    const int steps = series_apply<N>(acc, r, mp.diag, mp.gram_scale2, mp.series, basis, r0, sh.mirror, lane);
     if (lane == 0) {
         left[g] = steps == 0;
         if (mp.series_steps) atomicAdd(mp.series_steps, (unsigned long long)steps);
@@ -1197,32 +1388,33 @@ __device__ __forceinline__ void series_body(int bx, int nbx, const int* __restri
     }
     dw += __shfl_xor(dw, 16);
     dw += __shfl_xor(dw, 32);
+    dw *= pow2_inverse(r0);
     asm volatile("" : "+v"(ln));  // the addresses again, for the same reason
     const int co = ln & 15, go = ln >> 4;
     if (mp.write_state && co < Q) {
         const float s = float(mp.sqm1);
-        float* fo = f + (long long)co * mp.nodes + g + 4 * go * mp.member_stride;
+        float* fo = f + (long long)co * mp.nodes + g + 4 * NT * go * mp.member_stride;
         bool bad = false;
 #pragma unroll
         for (int T = 0; T < NT; ++T)
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                if (16 * T + 4 * go + k >= M) continue;
+                if (NT * (4 * go + k) + T >= M) continue;
                 const float xa = float(xbar + double(fmaf(s, r[T][k], dw)));
                 bad |= !isfinite(xa);
-                fo[(16 * T + k) * mp.member_stride] = xa;
+                fo[(NT * k + T) * mp.member_stride] = xa;
             }
         if (bad) atomicOr(status, 1);
     }
 }
 
 template <int N, int PASSES>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_series_analysis(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_series_analysis(
     const int* __restrict__ loc_ptr, const int* __restrict__ loc_site, const float* __restrict__ loc_w,
     const float* __restrict__ dy, const float* __restrict__ dyo, float* __restrict__ f, MixedParams mp,
     int* __restrict__ status, unsigned char* __restrict__ left) {
     __shared__ __align__(16) SeriesShared<N> sh;
-    series_body<N, PASSES>(blockIdx.x, gridDim.x, loc_ptr, loc_site, loc_w, dy, dyo, f, mp, status, left, sh.basis);
+    series_body<N, PASSES>(blockIdx.x, gridDim.x, loc_ptr, loc_site, loc_w, dy, dyo, f, mp, status, left, sh);
 }
 
 template <int N, int PASSES>
@@ -1706,16 +1898,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 }
 
 template <int PASSES>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_series_analysis_group(MixedGroup G) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_series_analysis_group(
+    MixedGroup G) {
     int k = 0;
     while (k + 1 < G.n && int(blockIdx.x) >= G.t[k + 1].b0_finish) ++k;
     const MixedTask& T = G.t[k];
     const int bx = int(blockIdx.x) - T.b0_finish;
     __shared__ __align__(16) SeriesShared<64> sh;
     switch (T.N) {
-        case 16: series_body<16, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status, T.left, sh.basis); break;
-        case 32: series_body<32, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status, T.left, sh.basis); break;
-        default: series_body<64, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status, T.left, sh.basis); break;
+        case 16: series_body<16, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status,
+                                         T.left, *reinterpret_cast<SeriesShared<16>*>(&sh)); break;
+        case 32: series_body<32, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status,
+                                         T.left, *reinterpret_cast<SeriesShared<32>*>(&sh)); break;
+        default: series_body<64, PASSES>(bx, T.nb_finish, T.loc_ptr, T.loc_site, T.loc_w, T.dy, T.dyo, T.f, T.mp, T.status,
+                                         T.left, sh); break;
     }
 }
 
@@ -1797,7 +1993,8 @@ MixedParams mixed_params(const Ctx& c, unsigned long long* sweeps32, unsigned lo
     mp.chain = c.mix_chain;
     mp.write_state = 1;
     mp.series = c.d_series;
-    mp.series_scale = std::exp2(-float(std::ilogb(mp.diag)));
+    mp.gram_scale = std::exp2(std::floor(0.5f * float(5 - std::ilogb(mp.diag))));
+    mp.gram_scale2 = mp.gram_scale * mp.gram_scale;
     mp.series_steps = c.prof ? c.d_series_steps : nullptr;
     return mp;
 }

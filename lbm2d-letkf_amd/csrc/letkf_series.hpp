@@ -12,11 +12,12 @@
 // with the block per step.  Two full products (A^2 and T_2^2) and about 2.2 sqrt(kappa)
 // block products replace the Jacobi sweeps; nothing but matrix products is left.
 //
-// Products: v_mfma_f32_16x16x32_bf16 (x16 for one tile) with every operand split into
-// three bf16 parts (24 mantissa bits) and the six products of weight above 2^-24, FP32
-// accumulation: the FP32 matrix instructions take 2.7 times as long for the same bits.
-// Against 64 bits the products and the series leave an error of 1e-7 to 1e-6 of the
-// result (kappa up to 400), a tenth or less of what the split Gram matrix leaves.
+// Products: v_mfma_f32_16x16x32_f16 (x16 for one tile), every operand scaled by a power of
+// two into the range of f16 and split into two f16 parts (22 mantissa bits and the sign
+// of the rest), the three products of weight above 2^-22, FP32 accumulation.  Against 64
+// bits the products and the series leave an error of 1e-7 (kappa 20) to 1e-6 (kappa 300)
+// of the result, as the same with three bf16 parts and six products or with the FP32
+// matrix instructions does (which take 2 and 5 times as long): the FP32 sums set it.
 // An accumulator tile is an operand as it stands: lane (c, g) holds rows 16 T + 4 g + r,
 // r = 0..3, of column c, so summing over k in the order (T, g, r), the tile (K, J) of a
 // matrix is the B operand of K-block K and, the matrix being symmetric, the tile (K, I)
@@ -36,8 +37,8 @@ namespace lbmletkf {
 // 1, and the coefficients d_kj of both.
 constexpr int SERIES_CLASS0 = 80;     // quadruples of the header (first quadruple of each class)
 // The widest class lies where the eigensolve of the same kernel family costs as much: in
-// the mixed analysis at N = 64 a block product costs 1/110 of the warm-started sweeps
-// (kappa 2000), in FP64 1/4000 of them; there the table ends it (0.7 MB).
+// the mixed analysis at N = 64 a block product costs about 1/200 of the warm-started sweeps,
+// and the range of f16 ends the table (kappa 1022, a up to 64); in FP64 1/4000 of them; there the table ends it (0.7 MB).
 constexpr int SERIES_CLASSES32 = 40, SERIES_CLASSES64 = 64;  // kappa up to 1024 and 65536
 constexpr double SERIES_EPS32 = 3e-8, SERIES_EPS64 = 1e-13;
 
@@ -94,138 +95,171 @@ std::vector<T> series_table(int classes, double eps) {
 
 // ---- on the device ------------------------------------------------------------------
 namespace {
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float quiet_nan() { return __int_as_float(0x7fc00000); }
+
+// 2^(to - floor(log2 x)), the power of two that brings x > 0 to [2^to, 2^(to+1)), its
+// exponent within +-100; 1 for x = 0 or not finite
+__device__ __forceinline__ float pow2_scale(float x, int to) {
+    const int ex = int((__float_as_uint(x) >> 23) & 255u);
+    const int k = min(100, max(-100, to + 127 - ex));
+    return ex == 0 || ex == 255 ? 1.f : __int_as_float((k + 127) << 23);
+}
+__device__ __forceinline__ float pow2_inverse(float s) { return __int_as_float((254 << 23) - __float_as_int(s)); }
+
+// x = p0 + p1 to 22 bits, each f16 (rounded to nearest), for a pair of values
+__device__ __forceinline__ void split_pair(float a, float b, f16x2& p0, f16x2& p1) {
+    p0 = __builtin_convertvector(f32x2{a, b}, f16x2);
+    float m1 = -1.f;
+    asm("" : "+s"(m1));  // a product, for v_fma_mix_f32: a subtraction would convert p0 first
+    p1 = __builtin_convertvector(f32x2{fmaf(float(p0[0]), m1, a), fmaf(float(p0[1]), m1, b)}, f16x2);
+}
 
 // Operands of one K-block: two accumulator tiles (32 values of k), or the only one of a
 // 16 x 16 problem.
 template <int N>
 struct SeriesOp {
     static constexpr int TILES = N >= 32 ? 2 : 1;
-    typedef bf16x8 vec;
+    typedef f16x8 vec;
 };
 template <>
 struct SeriesOp<16> {
     static constexpr int TILES = 1;
-    typedef bf16x4 vec;
+    typedef f16x4 vec;
 };
 
-__device__ __forceinline__ f32x4 series_mfma(bf16x8 a, bf16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+__device__ __forceinline__ f32x4 series_mfma(f16x8 a, f16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ f32x4 series_mfma(bf16x4 a, bf16x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0,
-                                                     0, 0);
+__device__ __forceinline__ f32x4 series_mfma(f16x4 a, f16x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
 }
 
-// x = p0 + p1 + p2, each bf16 (rounded to nearest), for a pair of values
-__device__ __forceinline__ void split_pair(float a, float b, bf16x2 (&p)[3]) {
+__device__ __forceinline__ void split_tiles(const f32x4* t, f16x8 (&p)[2]) {
+    f16x2 q[4][2];
 #pragma unroll
-    for (int s = 0; s < 3; ++s) {
-        p[s] = __builtin_convertvector(f32x2{a, b}, bf16x2);
-        if (s < 2) {
-            const unsigned bits = __builtin_bit_cast(unsigned, p[s]);
-            a -= __builtin_bit_cast(float, bits << 16);
-            b -= __builtin_bit_cast(float, bits & 0xffff0000u);
-        }
-    }
-}
-__device__ __forceinline__ void split_tiles(const f32x4* t, bf16x8 (&p)[3]) {
-    bf16x2 q[4][3];
+    for (int k = 0; k < 4; ++k) split_pair(t[k / 2][2 * (k % 2)], t[k / 2][2 * (k % 2) + 1], q[k][0], q[k][1]);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) split_pair(t[k / 2][2 * (k % 2)], t[k / 2][2 * (k % 2) + 1], q[k]);
-#pragma unroll
-    for (int s = 0; s < 3; ++s)
+    for (int s = 0; s < 2; ++s)
         p[s] = __builtin_shufflevector(__builtin_shufflevector(q[0][s], q[1][s], 0, 1, 2, 3),
                                        __builtin_shufflevector(q[2][s], q[3][s], 0, 1, 2, 3), 0, 1, 2, 3, 4, 5, 6, 7);
 }
-__device__ __forceinline__ void split_tiles(const f32x4* t, bf16x4 (&p)[3]) {
-    bf16x2 q[2][3];
+__device__ __forceinline__ void split_tiles(const f32x4* t, f16x4 (&p)[2]) {
+    f16x2 q[2][2];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) split_pair(t[0][2 * k], t[0][2 * k + 1], q[k]);
+    for (int k = 0; k < 2; ++k) split_pair(t[0][2 * k], t[0][2 * k + 1], q[k][0], q[k][1]);
 #pragma unroll
-    for (int s = 0; s < 3; ++s) p[s] = __builtin_shufflevector(q[0][s], q[1][s], 0, 1, 2, 3);
+    for (int s = 0; s < 2; ++s) p[s] = __builtin_shufflevector(q[0][s], q[1][s], 0, 1, 2, 3);
 }
 
-// c + a b over one K-block, the small products first
+// the products of c += a b, the small ones first: 0, 1, 2.  Callers go through all their
+// tiles with one product before the next, as a matrix instruction that adds to the result
+// of the one before waits for it.
 template <class V>
-__device__ __forceinline__ f32x4 series_fma(const V (&a)[3], const V (&b)[3], f32x4 c) {
-    c = series_mfma(a[0], b[2], c);
-    c = series_mfma(a[2], b[0], c);
-    c = series_mfma(a[1], b[1], c);
-    c = series_mfma(a[0], b[1], c);
-    c = series_mfma(a[1], b[0], c);
-    return series_mfma(a[0], b[0], c);
+__device__ __forceinline__ f32x4 series_fma(int product, const V (&a)[2], const V (&b)[2], f32x4 c) {
+    return product == 0   ? series_mfma(a[0], b[1], c)
+           : product == 1 ? series_mfma(a[1], b[0], c)
+                          : series_mfma(a[0], b[0], c);
+}
+
+// The transpose of a tile, through LDS: lane (c, g) writes rows 4 g .. 4 g + 3 of column c
+// and reads column c of rows 4 g + r (a column takes 20 words: no bank conflicts).  The
+// matrices here are symmetric: computed are their tiles on and above the diagonal, and
+// these 8 LDS instructions per tile below it stand against 6 matrix instructions of 16
+// cycles in a square and about 18 in a Gram matrix of 190 observations.
+constexpr int MIRROR_TILE = 16 * 20;
+// orders the LDS accesses of one wavefront, which the hardware executes in order
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ f32x4 transpose_tile(f32x4 x, float* lds, int lane) {
+    const int c = lane & 15, g = lane >> 4;
+    wave_lds_fence();  // (the reads before)
+    *reinterpret_cast<f32x4*>(lds + c * 20 + 4 * g) = x;
+    wave_lds_fence();
+    f32x4 y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = lds[(4 * g + r) * 20 + c];
+    return y;
 }
 
 // a symmetric matrix as operands: K-block kb, tile column j
 template <int N>
 struct SeriesMat {
     static constexpr int NT = N / 16, KB = NT / SeriesOp<N>::TILES;
-    typename SeriesOp<N>::vec p[KB][NT][3];
-    // from its tiles (K NT + J) scaled by s
-    __device__ __forceinline__ void set(const f32x4* t, float scale) {
+    typename SeriesOp<N>::vec p[KB][NT][2];
+    // from its tiles (I NT + J) with I <= J
+    __device__ __forceinline__ void set(const f32x4* t, float* lds, int lane) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
                 f32x4 x[SeriesOp<N>::TILES];
 #pragma unroll
-                for (int h = 0; h < SeriesOp<N>::TILES; ++h) x[h] = t[(kb * SeriesOp<N>::TILES + h) * NT + j] * scale;
+                for (int h = 0; h < SeriesOp<N>::TILES; ++h) {
+                    const int i = kb * SeriesOp<N>::TILES + h;
+                    x[h] = i <= j ? t[i * NT + j] : transpose_tile(t[j * NT + i], lds, lane);
+                }
                 split_tiles(x, p[kb][j]);
                 // opaque: under register pressure the compiler would sink the split into
                 // the loop that uses it
 #pragma unroll
-                for (int s = 0; s < 3; ++s) asm volatile("" : "+v"(p[kb][j][s]));
+                for (int s = 0; s < 2; ++s) asm volatile("" : "+v"(p[kb][j][s]));
                 __builtin_amdgcn_sched_barrier(0);
             }
     }
-    // its tile (K, J), exactly the sum of the parts
-    __device__ __forceinline__ f32x4 tile(int K, int J) const {
-        f32x4 x;
+    // k times its tile (K, J), plus y
+    __device__ __forceinline__ f32x4 axpy_tile(int K, int J, float k, f32x4 y) const {
         const int kb = K / SeriesOp<N>::TILES, h = 4 * (K % SeriesOp<N>::TILES);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            x[r] = float(p[kb][J][0][h + r]) + (float(p[kb][J][1][h + r]) + float(p[kb][J][2][h + r]));
-        return x;
+            y[r] = fmaf(float(p[kb][J][0][h + r]), k, fmaf(float(p[kb][J][1][h + r]), k, y[r]));
+        return y;
     }
-    // d = this * this
+    // d = this * this, the tiles on and above the diagonal
     __device__ __forceinline__ void square(f32x4* d) const {
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                f32x4 c{0.f, 0.f, 0.f, 0.f};
+            for (int j = i; j < NT; ++j) d[i * NT + j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int kb = 0; kb < KB; ++kb) c = series_fma(p[kb][i], p[kb][j], c);
-                d[i * NT + j] = c;
-                __builtin_amdgcn_sched_barrier(0);
-            }
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int s = 0; s < 3; ++s)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+#pragma unroll
+                    for (int j = i; j < NT; ++j)
+                        d[i * NT + j] = series_fma(s, p[kb][i], p[kb][j], d[i * NT + j]);
+        __builtin_amdgcn_sched_barrier(0);
     }
-    // c += this * (s v) for a block of sixteen columns v
-    __device__ __forceinline__ void times(const f32x4 (&v)[NT], float s, f32x4 (&c)[NT]) const {
+    // c += this * (f v) for a block of sixteen columns v
+    __device__ __forceinline__ void times(const f32x4 (&v)[NT], float f, f32x4 (&c)[NT]) const {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
             f32x4 x[SeriesOp<N>::TILES];
 #pragma unroll
-            for (int h = 0; h < SeriesOp<N>::TILES; ++h) x[h] = v[kb * SeriesOp<N>::TILES + h] * s;
-            typename SeriesOp<N>::vec b[3];
+            for (int h = 0; h < SeriesOp<N>::TILES; ++h) x[h] = v[kb * SeriesOp<N>::TILES + h] * f;
+            typename SeriesOp<N>::vec b[2];
             split_tiles(x, b);
 #pragma unroll
-            for (int i = 0; i < NT; ++i) c[i] = series_fma(p[kb][i], b, c[i]);
+            for (int s = 0; s < 3; ++s)
+#pragma unroll
+                for (int i = 0; i < NT; ++i) c[i] = series_fma(s, p[kb][i], b, c[i]);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 };
 
-// The four vectors V_j, in registers, or where a matrix fills those (N = 64), in LDS as
-// [j][T][lane].
+// The four vectors V_j, in registers, or where a matrix fills those (N = 64), V_3 and a
+// quarter of V_2 in registers and the others in LDS as [j][T][lane]: with the tile of
+// transpose_tile 12.5 KB, and so three wavefronts per SIMD (LDS is allocated in 1.25 KB).
 template <int N>
 struct SeriesBasis {
     static constexpr int NT = N / 16;
@@ -240,36 +274,58 @@ struct SeriesBasis {
 template <>
 struct SeriesBasis<64> {
     static constexpr int NT = 4;
+    f32x4 v3[NT], v2;
     f32x4* at;
     __device__ __forceinline__ SeriesBasis(float* lds, int lane) : at(reinterpret_cast<f32x4*>(lds) + lane) {}
     __device__ __forceinline__ void put(int j, const f32x4 (&x)[NT]) {
 #pragma unroll
-        for (int T = 0; T < NT; ++T) at[(j * NT + T) * 64] = x[T];
+        for (int T = 0; T < NT; ++T)
+            if (j == 3)
+                v3[T] = x[T];
+            else if (j == 2 && T == 3)
+                v2 = x[T];
+            else
+                at[(j * NT + T) * 64] = x[T];
     }
-    __device__ __forceinline__ f32x4 get(int j, int T) const { return at[(j * NT + T) * 64]; }
+    __device__ __forceinline__ f32x4 get(int j, int T) const {
+        return j == 3 ? v3[T] : j == 2 && T == 3 ? v2 : at[(j * NT + T) * 64];
+    }
 };
 
-// r := f(C) r for C = a I + A, A in the tiles `acc` (K NT + J; rows and columns past the
-// members zero): columns 0..8 of the block by x^(-1/2), column 9 by 1/x.  Returns the
-// number of block products taken, or 0, r untouched, where the spectrum is wider than the
-// widest class (or not finite).  A is taken times a power of two that brings a to [1, 2).
-// basis.get(0, .) holds the incoming r after a true return.  The scheduling barriers
-// keep the tiles in order: at N = 64 two matrices leave no registers to work ahead in.
+// r := f(C) r for C = a I + A, acc holding scale_a A in its tiles I NT + J with I <= J (rows
+// and columns past the members zero): columns 0..8 of the block by x^(-1/2), column 9 by
+// 1/x.  Returns the number of block products taken, or 0, r untouched, where the spectrum
+// is wider than the widest class (or not finite).  basis.get(0, .) holds the incoming r
+// times r0 after a true return.  Ranges in f16: scale_a is a power of two that brings a to
+// [16, 64) (the largest entry of A stays below 1022 * 64; a wider spectrum overflows into
+// the false return); T_2 times 2^8; the vectors times 2^e, the power of two at or below
+// al but no less than 2^-13, on the way into a product, 2 T_4 times 2^-e, and the columns of r times the powers of
+// two (r0) that then bring their largest entries to [16, 32): the recurrence's vectors
+// exceed those at most 40-fold (the norm of a column, and five times that over all
+// classes).  The scheduling barriers keep the tiles in order: at N = 64 two matrices leave
+// few registers to work ahead in.
 template <int N>
 __device__ __forceinline__ int series_apply(const f32x4* acc, f32x4 (&r)[N / 16], float a_in, float scale_a,
-                                            const float4* __restrict__ table, SeriesBasis<N>& basis, int lane) {
+                                            const float4* __restrict__ table, SeriesBasis<N>& basis, float& r0,
+                                            float* mirror, int lane) {
     constexpr int NT = N / 16;
     const float a = a_in * scale_a;
     SeriesMat<N> m;
-    m.set(acc, scale_a);
+    m.set(acc, mirror, lane);
     f32x4 sq[NT * NT];
     m.square(sq);
     // lambda_max(A) <= ||A^2||_F^(1/2) (at most rank^(1/4) too wide)
-    float ss = 0.f;
+    float ss = 0.f, st = 0.f;
 #pragma unroll
-    for (int t = 0; t < NT * NT; ++t)
+    for (int I = 0; I < NT; ++I)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) ss = fmaf(sq[t][k], sq[t][k], ss);
+        for (int J = I; J < NT; ++J)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float x = sq[I * NT + J][k];
+                (I == J ? ss : st) = fmaf(x, x, I == J ? ss : st);
+            }
+    ss += 2.f * st;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
     const float kappa = 1.f + 1.0001f * __builtin_amdgcn_sqrtf(__builtin_amdgcn_sqrtf(ss)) / a;
@@ -277,13 +333,24 @@ __device__ __forceinline__ int series_apply(const f32x4* acc, f32x4 (&r)[N / 16]
     const int cl = __builtin_amdgcn_readfirstlane(max(1, int(ceilf(4.f * log2f(kappa)))));
     const float lam = a * (exp2f(0.25f * float(cl)) - 1.f);
     const float al = 2.f / lam;  // x = al A - 1
+    const float inv_e = fminf(pow2_scale(al, 0), 0x1p13f), pow_e = pow2_inverse(inv_e);
     const float4 hd = table[cl];
     const int first = __builtin_amdgcn_readfirstlane(int(hd.x));
     const int K = __builtin_amdgcn_readfirstlane(int(hd.y));
 
     // V_0 = r, V_1 = x V_0, V_j = 2 x V_{j-1} - V_{j-2}
     {
+        float big = 0.f;
+#pragma unroll
+        for (int T = 0; T < NT; ++T)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) big = fmaxf(big, fabsf(r[T][k]));
+        big = fmaxf(big, __shfl_xor(big, 16));
+        big = fmaxf(big, __shfl_xor(big, 32));
+        r0 = pow2_scale(big * pow_e, 4);
         f32x4 v[NT];
+#pragma unroll
+        for (int T = 0; T < NT; ++T) r[T] *= r0;
         basis.put(0, r);
 #pragma unroll
         for (int T = 0; T < NT; ++T) v[T] = -r[T];
@@ -303,27 +370,30 @@ __device__ __forceinline__ int series_apply(const f32x4* acc, f32x4 (&r)[N / 16]
     // T_2(x) = 2 al^2 A^2 - 4 al A + I, then Y = T_4 = 2 T_2^2 - I; the recurrence takes 2 Y
     __builtin_amdgcn_sched_barrier(0);
     const int c = lane & 15, g = lane >> 4;
-    const float k2 = 2.f * al * al, k1 = -4.f * al;
+    const float k2 = 0x1p9f * al * al, k1 = -0x1p10f * al;
 #pragma unroll
     for (int I = 0; I < NT; ++I)
 #pragma unroll
-        for (int J = 0; J < NT; ++J) {
-            const f32x4 x = m.tile(I, J);
+        for (int J = I; J < NT; ++J) {
+            f32x4& x = sq[I * NT + J];
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                sq[I * NT + J][k] = fmaf(k2, sq[I * NT + J][k], fmaf(k1, x[k], I == J && 4 * g + k == c ? 1.f : 0.f));
+            for (int k = 0; k < 4; ++k) x[k] = I == J ? fmaf(k2, x[k], 4 * g + k == c ? 0x1p8f : 0.f) : k2 * x[k];
+            x = m.axpy_tile(I, J, k1, x);
             __builtin_amdgcn_sched_barrier(0);
         }
-    m.set(sq, 1.f);
+    m.set(sq, mirror, lane);
     m.square(sq);
+    const float q2 = 0x1p-14f * inv_e;
 #pragma unroll
     for (int I = 0; I < NT; ++I)
 #pragma unroll
-        for (int J = 0; J < NT; ++J)
+        for (int J = I; J < NT; ++J)
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                sq[I * NT + J][k] = fmaf(4.f, sq[I * NT + J][k], I == J && 4 * g + k == c ? -2.f : 0.f);
-    m.set(sq, 1.f);
+            for (int k = 0; k < 4; ++k) {
+                const float x = sq[I * NT + J][k];
+                sq[I * NT + J][k] = I == J ? fmaf(q2, x, 4 * g + k == c ? -2.f * inv_e : 0.f) : q2 * x;
+            }
+    m.set(sq, mirror, lane);
 
     // Clenshaw: B_k = Q_k + 2 Y B_{k+1} - B_{k+2}, Q_k = sum_j d_kj V_j; result Q_0 + Y B_1 - B_2
     const float4* coef = table + first + (c == 9 ? 1 : 0);
@@ -337,27 +407,32 @@ __device__ __forceinline__ int series_apply(const f32x4* acc, f32x4 (&r)[N / 16]
         }
     }
     float4 d = coef[2 * (K - 2)];
-#pragma unroll 1
-    for (int k = K - 2; k >= 0; --k) {
+    // old := Q_k + 2 Y cur - old, in place: two steps per pass need no copies
+    auto step = [&](int k, const f32x4 (&cur)[NT], f32x4 (&old)[NT]) __attribute__((always_inline)) {
         const float4 dn = coef[2 * max(k - 1, 0)];
-        f32x4 q[NT];
 #pragma unroll
         for (int T = 0; T < NT; ++T) {
             const f32x4 x0 = basis.get(0, T), x1 = basis.get(1, T), x2 = basis.get(2, T), x3 = basis.get(3, T);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                q[T][e] = fmaf(d.x, x0[e], fmaf(d.y, x1[e], fmaf(d.z, x2[e], fmaf(d.w, x3[e], -b2[T][e]))));
+                old[T][e] = fmaf(d.x, x0[e], fmaf(d.y, x1[e], fmaf(d.z, x2[e], fmaf(d.w, x3[e], -old[T][e]))));
         }
-        m.times(b1, k > 0 ? 1.f : 0.5f, q);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) {
-            b2[T] = b1[T];
-            b1[T] = q[T];
-        }
+        m.times(cur, k > 0 ? pow_e : 0.5f * pow_e, old);
         d = dn;
+    };
+    int k = K - 2;
+#pragma unroll 1
+    for (; k > 0; k -= 2) {
+        step(k, b1, b2);
+        step(k - 1, b2, b1);
+    }
+    if (k == 0) {
+        step(0, b1, b2);
+#pragma unroll
+        for (int T = 0; T < NT; ++T) b1[T] = b2[T];
     }
     // f(C) = a^(-1/2) f(C / a), 1 / C = (1/a) 1 / (C / a)
-    const float scale = c == 9 ? 1.f / a_in : 1.f / sqrtf(a_in);
+    const float scale = (c == 9 ? 1.f / a_in : 1.f / sqrtf(a_in)) * pow2_inverse(r0);
 #pragma unroll
     for (int T = 0; T < NT; ++T) r[T] = b1[T] * scale;
     return K + 2;
