@@ -811,12 +811,17 @@ __device__ __forceinline__ float jacobi_fp32(float (&u)[N], float& sc, const flo
         a0 = fmaf(u[i], u[i], a0);
     }
     // keep the squared column norms below 1e18 (the range of the rotation
-    // formula): scale U by 2^-32 when needed, exactly, and undo it on output
+    // formula): when needed scale U, exactly, by the power of two that brings its largest
+    // element to [2^23, 2^24), and undo it on output
     float uscale = 1.f;
     if (wave_max(a0) > 1e18f) {
-        uscale = 0x1p32f;
+        float big = 0.f;
 #pragma unroll
-        for (int i = 0; i < N; ++i) u[i] *= 0x1p-32f;
+        for (int i = 0; i < N; ++i) big = fmaxf(big, fabsf(u[i]));
+        const float down = pow2_scale(wave_max(big), 23);
+        uscale = pow2_inverse(down);
+#pragma unroll
+        for (int i = 0; i < N; ++i) u[i] *= down;
     }
 
     // ---- 3. FP32 one-sided Jacobi ------------------------------------------------

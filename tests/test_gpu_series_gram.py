@@ -48,10 +48,10 @@ def test_gram_shapes(lb, orc, M, obs_vars, stride, cutoff, passes):
 
 
 @pytest.mark.parametrize("M", [8, 32])
-@pytest.mark.parametrize("sigma", [1e-7])
+@pytest.mark.parametrize("sigma", [1e-7, 1e-12])
 def test_past_the_range(lb, M, sigma):
-    # rows of dY past the range of f16: the sweeps take every gridpoint, as when all are
-    # dumped
+    # rows of dY past the range of f16, and a matrix whose squared columns pass FP32's: the
+    # sweeps take every gridpoint, as when all are dumped, and stay finite
     cfg = small_cfg(lb, "baseline", n=64, obs_stride=4, loc_scale=3.0, loc_cutoff=9.0, obs_sigma_u=sigma)
     cfg.ny = 40
     print(f"case: range M={M} sigma={sigma}", flush=True)
@@ -68,3 +68,16 @@ def test_past_the_range(lb, M, sigma):
     assert np.isfinite(fa).all()
     np.testing.assert_array_equal(fa, fs)
 
+
+def test_density_that_cancels(lb):
+    # populations of either sign whose sum is exactly zero are observed with a finite
+    # velocity, c (-0.25 - 0.25) over half a unit in the last place of 0.25
+    cfg = small_cfg(lb, "baseline", n=64, obs_stride=8, loc_scale=3.0, loc_cutoff=7.0)
+    with lb.Context(cfg, 1) as ctx:
+        f = np.full((9, 64, 64), 1.0 / 9, np.float32)
+        f[:, 16, 24] = 0.0
+        f[0, 16, 24], f[8, 16, 24] = 0.25, -0.25
+        ctx.set_state(0, f)
+        y = ctx.observe(0, seed=11, counter=3, noise=False)
+    assert np.isfinite(y).all()
+    assert np.abs(y).max() == np.float32(cfg.c * 0.5 / 2.0**-27)
