@@ -94,7 +94,7 @@ struct Ctx {
 
     // device status word: bit 0 = NaN in analysis
     int* d_status = nullptr;
-    int* h_status = nullptr;      // pinned
+    int* h_status = nullptr;  // pinned: the word as of the last wait
 
     // observation network and local sets (CSR over gridpoints)
     bool obs_ready = false;
