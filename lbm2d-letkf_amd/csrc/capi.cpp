@@ -1901,7 +1901,9 @@ int lbmletkf_autotune(lbmletkf_ctx* ctx, const char* cache_path, char* report, i
                 return st;
             std::snprintf(buf, sizeof buf, " %d:%.1f", ch, us);
             rep += buf;
-            if (us < best) {
+            // a longer chain has to be faster by more than launches of one length differ:
+            // where the series takes every gridpoint all lengths cost the same
+            if (us < 0.97 * best) {
                 best = us;
                 best_chain = ch;
             }
