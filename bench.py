@@ -8,12 +8,12 @@ LBM steps of all 64 members + one LETKF analysis at all 65,536 gridpoints.
 The nature run and its observations for every cycle are generated first and kept
 in HBM; the timed region covers K cycles of the ensemble only (the reference's
 `forecast` + `DA` timers, src/main.cu:95-115).  The variants:
-plain (per-member LBM launches, FP32 Gram, FP64 two-sided Jacobi, eager launches) at
-the preset's eigensolver tolerance (1e-10) and at the reference's (syevj tolerance
-1e-6, src/util/cu_matrix_eigensolver_wrapper.hpp:192,202), and mixed (all members'
-LBM steps in one launch, one fused analysis kernel -- split-bf16 MFMA Gram, FP32
-one-sided Jacobi, FP64 eigenvalue coefficients, FP32 MFMA update -- each cycle
-replayed from a hipGraph).  `value` is the mixed variant's DA cycles/s.  The
+plain (FP32 Gram, FP64 matrix-core series with a two-sided Jacobi behind it, eager
+launches) at the preset's eigensolver tolerance (1e-10) and at the reference's (syevj
+tolerance 1e-6, src/util/cu_matrix_eigensolver_wrapper.hpp:192,202), which only the
+Jacobi reads, and mixed (Gram and the update by Chebyshev series on the matrix cores with
+operands in two f16 parts, FP32 sweeps for gridpoints too badly conditioned for it; each
+cycle replayed from a hipGraph).  `value` is the mixed variant's DA cycles/s.  The
 analysis RMSE of each variant is taken at the observation time after the timed
 cycles; a few further cycles with phase timing on give the per-kernel breakdown.
 
@@ -41,8 +41,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-FP32_PEAK_TFLOPS = 157.3      # published FP32 vector peak (counts packed FP32 issue)
-FP32_UNPACKED_TFLOPS = 78.6   # the same without packed FP32, which this build never emits
+FP32_PEAK_TFLOPS = 157.3      # published FP32 peak, vector (counting packed issue) and matrix
 LBM_BYTES_PER_NODE_UPDATE = 72  # 9 x 4 B read + 9 x 4 B written
 
 
@@ -183,7 +182,11 @@ def bench_variant(lb, hip, cfg, variant, M, K, W, P, obs, truth, n_obs, log, rep
         ens.forecast(steps)
         ens.analysis_device(yo(cc))
     ens.synchronize()
-    phases = {ph: ens.profile_read(ph) for ph in ("forecast", "obs", "gram", "solve", "finish", "solve_fp64")}
+    phases = {ph: ens.profile_read(ph) for ph in ("forecast", "obs", "gram", "solve", "finish", "solve_fp64",
+                                                 "solve_series")}
+    # scalar observations of a gridpoint's local set, over a sample of the grid
+    n_sites, n_all = ens.obs_count()
+    local_obs = float(np.mean([len(ens.local_obs(g)[0]) for g in range(0, cfg.nx * cfg.ny, 509)])) * n_all / n_sites
     ens.close()
     ws = sorted(walls)
     wall = ws[len(ws) // 2]
@@ -195,7 +198,7 @@ def bench_variant(lb, hip, cfg, variant, M, K, W, P, obs, truth, n_obs, log, rep
     return dict(wall=wall, walls=walls, iqr_cycles_per_s=[K / q3, K / q1], event_s=float(np.median(evs)) / 1e3,
                 phases=phases, stats=stats, steps=steps, state=final_state, yo_index=ca, prof_cycles=P,
                 variant="plain" if variant == lb.VARIANT_PLAIN else "mixed", tuning=tuning, K=K,
-                jacobi_tol=cfg.jacobi_tol, closure="smagorinsky" if closure is None else "mlp")
+                local_obs=local_obs, jacobi_tol=cfg.jacobi_tol, closure="smagorinsky" if closure is None else "mlp")
 
 
 def rmse_probe(lb, cfg, M, n_cycles, obs, truth, n_obs):
@@ -255,30 +258,33 @@ def kernel_table(r, M, nodes):
                            peak=HBM_PEAK_GBS, bound="hbm", share=sec)
     sec, n, sweeps = r["phases"]["solve"]
     sweeps_gp = sweeps / (nodes * P) if P else 0.0
+    # block products of the series per gridpoint, and the flops they and its two squares
+    # (of symmetric matrices, half of which is computed) are worth: a block has ten vectors
+    steps_gp = r["phases"]["solve_series"][2] / (nodes * P) if P else 0.0
+    series_flops = (2 * M * M * (M + 1) + steps_gp * 2 * M * M * 10) * nodes if steps_gp else 0.0
     if r["variant"] == "mixed":
-        # the fused analysis kernel is bound by its FP32 vector ALU (the one-sided
-        # sweeps).  Algorithmic flops of a one-sided sweep: N-1 rounds x N columns x
-        # (N FMA for the pair inner product + N FMA for the update) ~ 4 N^3 (N = M = 64).
-        # The two-sided count (M(M-1)/2 rotations x 18 M per sweep) is given beside it.
-        t = sec / max(n, 1)
-        flops_own = 4.0 * M**3 * sweeps_gp * nodes
-        flops_2s = M * (M - 1) / 2 * 18.0 * M * sweeps_gp * nodes
+        # Bound by instruction issue, vector and matrix instructions together.  Counted in
+        # FP32: a product of f16 parts is three on the matrix cores, against the published
+        # FP32 peak.  The Gram matrix of the local observations is symmetric as well.  What
+        # the sweeps took (gridpoints too badly conditioned for the series) is not counted.
+        t = sec / max(P, 1)  # (two launches: the series, and the sweeps for what it left)
+        gram_flops = M * (M + 1) * r["local_obs"] * nodes
+        own = series_flops + gram_flops
         out["letkf_analysis"] = dict(
-            avg_ms=t * 1e3, achieved=flops_own / t / 1e12 if t else 0.0, unit="TFLOP/s",
-            peak=FP32_PEAK_TFLOPS, bound="valu",
-            kernel="k_mixed_analysis<64, 3> (gather + split-bf16 MFMA Gram + FP32 one-sided sweeps + "
-                   "FP64 coefficients + FP32 MFMA update)",
-            flop_count="one-sided Jacobi: 4 N^3 per sweep per gridpoint x measured sweeps",
-            peak_unpacked_fp32=FP32_UNPACKED_TFLOPS,
-            frac_of_unpacked_fp32=(flops_own / t / 1e12 / FP32_UNPACKED_TFLOPS) if t else 0.0,
-            achieved_two_sided_count=flops_2s / t / 1e12 if t else 0.0,
-            frac_two_sided_count=(flops_2s / t / 1e12 / FP32_PEAK_TFLOPS) if t else 0.0,
+            avg_ms=t * 1e3, achieved=own / t / 1e12 if t else 0.0, unit="TFLOP/s",
+            peak=FP32_PEAK_TFLOPS, bound="issue",
+            kernel="k_series_analysis<64, 3> (gather + Gram + Chebyshev series, f16 parts on the matrix cores)",
+            flop_count="FP32 flops per gridpoint: Gram M (M + 1) per local observation, two symmetric squares, "
+                       "2 M^2 x 10 per measured block product",
+            block_products_per_gridpoint=steps_gp, local_obs_per_gridpoint=r["local_obs"],
             sweeps_per_gridpoint=sweeps_gp, fp64_sweeps_per_gridpoint=0.0, share=sec)
     else:
-        flops = 9.0 * M**3 * sweeps  # two-sided rotation update (12M) + V update (6M) per rotation
-        out["letkf_solve"] = dict(avg_ms=sec / max(n, 1) * 1e3, achieved=flops / sec / 1e12 if sec else 0.0,
-                                  unit="TFLOP/s", peak=FP64_PEAK_TFLOPS, bound="valu",
-                                  engine="fp64 vector ALU + LDS (two-sided Jacobi)",
+        # counted are the rotations of what the series left: the two-sided update (12M) and
+        # the V update (6M) of each; the FP64 series keeps no count
+        flops = 9.0 * M**3 * sweeps
+        out["letkf_solve"] = dict(avg_ms=sec / max(P, 1) * 1e3, achieved=flops / sec / 1e12 if sec else 0.0,
+                                  unit="TFLOP/s", peak=FP64_PEAK_TFLOPS, bound="mfma",
+                                  engine="fp64 matrix cores (series)",
                                   sweeps_per_gridpoint=sweeps_gp, share=sec)
     sec, n, pobs = r["phases"]["gram"]
     if n:
@@ -540,9 +546,8 @@ def main():
     dom_name = max(kern, key=lambda k: kern[k]["share"])
     dom = kern[dom_name]
     tune = head.get("tuning") or [1, 8]
-    solve_wg = (nodes + tune[1] - 1) // tune[1]
     mixed = head["variant"] == "mixed"
-    traffic_ana = measured_traffic("k_mixed_analysis<64, 3>", solve_wg) if mixed else None
+    traffic_ana = measured_traffic("k_series_analysis<64, 3>", (nodes + 7) // 8 * 8) if mixed else None
     if tune[0] <= -200:
         lbm_kernel = "k_lbm_rows3<%d, %d>" % (-tune[0] - 200, 256 if cfg.nx == 256 else 0)
         lbm_wg = (cfg.ny // (-tune[0] - 200)) * M
@@ -560,8 +565,7 @@ def main():
                 traffic_unit="bytes per launch, rocprofv3 FETCH_SIZE x2 + WRITE_SIZE "
                              "(profiles/hbm_traffic_256x256_M64.md)",
                 avg_launch_ms=dom["avg_ms"], share_of_cycle=dom["share"])
-    for key in ("flop_count", "peak_unpacked_fp32", "frac_of_unpacked_fp32", "achieved_two_sided_count",
-                "frac_two_sided_count", "sweeps_per_gridpoint"):
+    for key in ("flop_count", "block_products_per_gridpoint", "local_obs_per_gridpoint", "sweeps_per_gridpoint"):
         if key in dom:
             roof[key] = dom[key]
     lbm = kern["lbm_step"]
@@ -577,9 +581,9 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": ("FP32 LBM; analysis: split-bf16x3 MFMA Gram (FP32 accumulation), FP32 one-sided Jacobi "
-                  "(0 FP64 sweeps), FP64 eigenvalue norms and coefficients, FP32 MFMA W.Xb update") if mixed
-                 else "FP32 LBM; FP32 Gram; FP64 two-sided Jacobi and transform",
+        "dtype": ("FP32 LBM; analysis: MFMA Gram and Chebyshev series, operands in two f16 parts (22 bits), FP32 "
+                  "accumulation, FP32 sweeps where ill-conditioned, FP64 ensemble mean") if mixed
+                 else "FP32 LBM; FP32 Gram; FP64 series or two-sided Jacobi and transform",
         "data": "synthetic",
         "config": {"workload": "LETKF OSSE 256x256, M=64 members, 100 LBM steps per DA cycle, "
                                "(u,v) every 8th node, Gaussian L=12 cutoff 43.8, beta=1.1",
@@ -593,7 +597,7 @@ def main():
                          "analysis_rmse": r["stats"][0], "analysis_spread": r["stats"][1],
                          "tuning_lbm_tiles_per_block_and_chain": r["tuning"],
                          "phase_ms_per_cycle": {p: r["phases"][p][0] / P * 1e3 for p in r["phases"]
-                                                if p != "solve_fp64"}}
+                                                if p not in ("solve_fp64", "solve_series")}}
                      for k, r in res.items()},
         "roofline": roof,
         "roofline_lbm": dict(kernel=lbm_kernel, bound="hbm", achieved=lbm["achieved"], peak=HBM_PEAK_GBS,

@@ -1337,8 +1337,9 @@ int lbmletkf_profile_enable(lbmletkf_ctx* ctx, int on) {
     }
     if (!c->d_sweeps) HIP_TRY(c, dalloc(&c->d_sweeps, 1));
     if (!c->d_sweeps64) HIP_TRY(c, dalloc(&c->d_sweeps64, 1));
-    if (!c->d_series_steps) HIP_TRY(c, dalloc(&c->d_series_steps, 1));
-    HIP_TRY(c, hipMemset(c->d_series_steps, 0, sizeof(unsigned long long)));
+    constexpr size_t series_words = size_t(SERIES_SLOTS) * SERIES_SLOT_STRIDE;
+    if (!c->d_series_steps) HIP_TRY(c, dalloc(&c->d_series_steps, series_words));
+    HIP_TRY(c, hipMemset(c->d_series_steps, 0, sizeof(unsigned long long) * series_words));
     HIP_TRY(c, hipMemset(c->d_sweeps, 0, sizeof(unsigned long long)));
     HIP_TRY(c, hipMemset(c->d_sweeps64, 0, sizeof(unsigned long long)));
     c->prof = on != 0;
@@ -1361,8 +1362,13 @@ int lbmletkf_profile_read(lbmletkf_ctx* ctx, const char* phase, double* seconds,
         // block products of the series, or FP64 sweeps, of the MIXED variant (their time is
         // part of "solve")
         unsigned long long sw = 0;
-        const unsigned long long* d = series ? c->d_series_steps : c->d_sweeps64;
-        if (d) HIP_TRY(c, hipMemcpy(&sw, d, sizeof(sw), hipMemcpyDeviceToHost));
+        if (series && c->d_series_steps) {
+            std::vector<unsigned long long> part(size_t(SERIES_SLOTS) * SERIES_SLOT_STRIDE);
+            HIP_TRY(c, hipMemcpy(part.data(), c->d_series_steps, sizeof(sw) * part.size(), hipMemcpyDeviceToHost));
+            for (int k = 0; k < SERIES_SLOTS; ++k) sw += part[size_t(k) * SERIES_SLOT_STRIDE];
+        } else if (!series && c->d_sweeps64) {
+            HIP_TRY(c, hipMemcpy(&sw, c->d_sweeps64, sizeof(sw), hipMemcpyDeviceToHost));
+        }
         if (seconds) *seconds = 0.0;
         if (launches) *launches = 0;
         if (work) *work = (long long)sw;

@@ -14,6 +14,9 @@ constexpr int Q = 9;
 constexpr int MAX_MEMBERS = 64;      // one wavefront of lanes per ensemble matrix
 constexpr int MAX_FORCE_MODES = 100; // src/data.cu:191-212 prunes to 100 modes
 constexpr int MIXED_GROUP_MAX = 8;   // contexts in one group launch
+// counters of the series' block products while profiling: one address would cost the
+// analysis of 256^2 gridpoints 0.2 ms of atomics
+constexpr int SERIES_SLOTS = 64, SERIES_SLOT_STRIDE = 16;
 // doubles per gridpoint of the transform dump (layout at Ctx::d_dump)
 __host__ __device__ constexpr long long dump_record(int M) { return 3LL * M * M + 2LL * M; }
 constexpr int LBM_TWO_STEP = 100;    // shape code offset of the two-step strips
@@ -159,7 +162,8 @@ struct Ctx {
     long long prof_work[PH_COUNT] = {};
     unsigned long long* d_sweeps = nullptr;    // Jacobi sweeps summed over gridpoints
     unsigned long long* d_sweeps64 = nullptr;  // MIXED: FP64 sweeps summed over gridpoints
-    unsigned long long* d_series_steps = nullptr;  // MIXED: block products of the series summed over gridpoints
+    unsigned long long* d_series_steps = nullptr;  // MIXED: block products of the series summed over gridpoints,
+                                                   // in SERIES_SLOTS parts, a cache line each
     int dump_kind = 0;  // 0: W, w, evals (plain); 1: V, d, b (mixed), assembled on the host
 
     // MIXED cycle (analysis + da_interval steps) as an instantiated hipGraph, one per

@@ -70,7 +70,7 @@ struct MixedParams {
     const float4* series;   // k_series_analysis: coefficients of the series (letkf_series.hpp)
     float gram_scale;       // k_series_analysis: the power of two applied to the rows of dY
     float gram_scale2;      // its square, which brings diag to [16, 64)
-    unsigned long long* series_steps;  // block products summed over gridpoints (may be null)
+    unsigned long long* series_steps;  // block products summed over gridpoints, in SERIES_SLOTS parts (may be null)
     unsigned long long* sweeps32;
     unsigned long long* sweeps64;
 };
@@ -1378,7 +1378,8 @@ __device__ __forceinline__ void series_body(int bx, int nbx, const int* __restri
     const int steps = series_apply<N>(acc, r, mp.diag, mp.gram_scale2, mp.series, basis, r0, sh.mirror, lane);
     if (lane == 0) {
         left[g] = steps == 0;
-        if (mp.series_steps) atomicAdd(mp.series_steps, (unsigned long long)steps);
+        if (mp.series_steps)
+            atomicAdd(mp.series_steps + (bx % SERIES_SLOTS) * SERIES_SLOT_STRIDE, (unsigned long long)steps);
     }
     if (steps == 0) return;
     // dX w = sum_k dX[k] w[k], w = C^-1 b in column 9 (row_newbcast:9)
