@@ -42,6 +42,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
 FP32_PEAK_TFLOPS = 157.3      # published FP32 peak, vector (counting packed issue) and matrix
+F16_PEAK_TFLOPS = 2500.0      # published dense f16 matrix peak
 LBM_BYTES_PER_NODE_UPDATE = 72  # 9 x 4 B read + 9 x 4 B written
 
 
@@ -248,6 +249,8 @@ def kernel_table(r, M, nodes):
     sec, n, work = r["phases"]["forecast"]
     n_steps = r["steps"] * P
     spl = lbm_steps_per_launch(r.get("tuning"))
+    if r.get("tuning") and r["tuning"][0] == 1:  # the library's rule: from its launches
+        spl = max(1, round(n_steps / max(n, 1)))
     avg = sec / n_steps  # one forecast step (all launches of the step)
     # algorithmic HBM bytes of one launch: every population read once and written
     # once, whether the launch takes one step or two
@@ -263,18 +266,17 @@ def kernel_table(r, M, nodes):
     steps_gp = r["phases"]["solve_series"][2] / (nodes * P) if P else 0.0
     series_flops = (2 * M * M * (M + 1) + steps_gp * 2 * M * M * 10) * nodes if steps_gp else 0.0
     if r["variant"] == "mixed":
-        # Bound by instruction issue, vector and matrix instructions together.  Counted in
-        # FP32: a product of f16 parts is three on the matrix cores, against the published
-        # FP32 peak.  The Gram matrix of the local observations is symmetric as well.  What
+        # Bound by instruction issue, vector and matrix instructions together.  A product
+        # counts once though it is three of f16 parts: against a third of the f16 peak.  The Gram matrix of the local observations is symmetric as well.  What
         # the sweeps took (gridpoints too badly conditioned for the series) is not counted.
         t = sec / max(P, 1)  # (two launches: the series, and the sweeps for what it left)
         gram_flops = M * (M + 1) * r["local_obs"] * nodes
         own = series_flops + gram_flops
         out["letkf_analysis"] = dict(
             avg_ms=t * 1e3, achieved=own / t / 1e12 if t else 0.0, unit="TFLOP/s",
-            peak=FP32_PEAK_TFLOPS, bound="issue",
+            peak=F16_PEAK_TFLOPS / 3, bound="issue",
             kernel="k_series_analysis<64, 3> (gather + Gram + Chebyshev series, f16 parts on the matrix cores)",
-            flop_count="FP32 flops per gridpoint: Gram M (M + 1) per local observation, two symmetric squares, "
+            flop_count="flops per gridpoint (each three on the f16 matrix cores): Gram M (M + 1) per local observation, two symmetric squares, "
                        "2 M^2 x 10 per measured block product",
             block_products_per_gridpoint=steps_gp, local_obs_per_gridpoint=r["local_obs"],
             sweeps_per_gridpoint=sweeps_gp, fp64_sweeps_per_gridpoint=0.0, share=sec)
@@ -555,16 +557,20 @@ def main():
         lbm_kernel, lbm_wg = "k_lbm_rows2<%d>" % (-tune[0] - 100), (cfg.ny // (-tune[0] - 100)) * M
     elif tune[0] < 0:
         lbm_kernel, lbm_wg = "k_lbm_rows<false, %d>" % -tune[0], (cfg.ny // -tune[0]) * M
+    elif tune[0] == 1:
+        lbm_kernel, lbm_wg = "the library's shape", 0
     else:
         lbm_kernel, lbm_wg = "k_lbm_fused<false>", cfg.nx // 64 * (cfg.ny // 16) * M // tune[0]
     traffic_lbm = measured_traffic(lbm_kernel, lbm_wg) if mixed else None
+    if dom_name == "lbm_step":
+        dom = dict(dom, kernel=lbm_kernel)
     roof = dict(kernel=dom.get("kernel", dom_name), bound=dom.get("bound", "hbm"), achieved=dom.get("achieved"),
                 peak=dom.get("peak"), unit=dom.get("unit"),
                 frac=(dom["achieved"] / dom["peak"]) if dom.get("peak") else None,
-                traffic=traffic_ana if dom_name == "letkf_analysis" else None,
+                traffic={"letkf_analysis": traffic_ana, "lbm_step": traffic_lbm}.get(dom_name),
                 traffic_unit="bytes per launch, rocprofv3 FETCH_SIZE x2 + WRITE_SIZE "
                              "(profiles/hbm_traffic_256x256_M64.md)",
-                avg_launch_ms=dom["avg_ms"], share_of_cycle=dom["share"])
+                avg_launch_ms=dom.get("avg_launch_ms", dom["avg_ms"]), share_of_cycle=dom["share"])
     for key in ("flop_count", "block_products_per_gridpoint", "local_obs_per_gridpoint", "sweeps_per_gridpoint"):
         if key in dom:
             roof[key] = dom[key]

@@ -1194,8 +1194,7 @@ __device__ __forceinline__ void series_gram_nv(int e0, int e1, int lane, const i
     entry(0, site, w);
     for (int b32 = 0; b32 < E; b32 += 32) {
         if (b32 % 64 == 0) {
-            // 24-bit product where dY, below 2^31 bytes, has rows of more than 2^7
-            at = int(N > 32 ? __umul24(site, row) : site * row);
+            at = int(site * row);
             ao = site * (NV * 4);
             sw = __builtin_amdgcn_sqrtf(w);
             entry(b32 + 64, site, w);

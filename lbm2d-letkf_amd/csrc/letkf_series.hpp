@@ -38,7 +38,8 @@ namespace lbmletkf {
 constexpr int SERIES_CLASS0 = 80;     // quadruples of the header (first quadruple of each class)
 // The widest class lies where the eigensolve of the same kernel family costs as much: in
 // the mixed analysis at N = 64 a block product costs about 1/200 of the warm-started sweeps,
-// and the range of f16 ends the table (kappa 1022, a up to 64); in FP64 1/4000 of them; there the table ends it (0.7 MB).
+// and the range of f16 ends it (kappa 1022, a up to 64); in FP64 1/4000 of the eigensolve,
+// and there the size of the table does (0.7 MB).
 constexpr int SERIES_CLASSES32 = 40, SERIES_CLASSES64 = 64;  // kappa up to 1024 and 65536
 constexpr double SERIES_EPS32 = 3e-8, SERIES_EPS64 = 1e-13;
 

@@ -351,9 +351,9 @@ class Context:
         return sec.value, n.value, w.value
 
     def set_tuning(self, lbm_tiles_per_block: int, mix_chain: int):
-        """LBM shape (k > 0 tiles per workgroup, -h row strips, -(100 + h) two-step
-        and -(200 + h) three-step row strips) and analysis chain length; see
-        lbmletkf_set_tuning."""
+        """LBM shape (1: the library's rule, k > 1 tiles per workgroup, -h row strips,
+        -(100 + h) two-step and -(200 + h) three-step row strips) and the chain length of
+        the analysis' sweeps; see lbmletkf_set_tuning."""
         self._ck(lib.lbmletkf_set_tuning(self.h, lbm_tiles_per_block, mix_chain))
 
     def get_tuning(self):
