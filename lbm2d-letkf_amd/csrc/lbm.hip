@@ -688,7 +688,7 @@ __global__ __launch_bounds__(BL_R * BL_R) void k_lbm_block(const float* __restri
 // The phase is reduced exactly in integers to a multiple of 2 pi / L, L the least
 // common multiple of nx and ny, so its sine and cosine come from a table of L entries
 // (a square grid: nx entries) instead of a reduction and a sincospif per node and mode:
-// 24 steps' draws and fields of a 256^2 grid take 4.6 + 21.6 us, against 19.7 us for each
+// 24 steps' draws and fields of a 256^2 grid take 4.6 + 18.2 us, against 19.7 us for each
 // step's with the phases reduced per node (same bits).  Where L is long the table stays in memory, and past
 // FORCE_TABLE_MAX entries the sines are formed in place.
 // ----------------------------------------------------------------------------
@@ -728,9 +728,21 @@ __device__ __forceinline__ int phase_step(int k, int a, int n) {
     return int(r < 0 ? r + n : r);
 }
 
+// the same without an integer division, for |k| <= 256 and n <= 2^14 (the product below
+// 2^21: its quotient in FP32 is off by one at most)
+__device__ __forceinline__ int phase_small(int k, int a, int n, float inv_n) {
+    const int num = __mul24(k, a - n / 2);
+    int r = num - __mul24(int(floorf(float(num) * inv_n)), n);
+    r = r < 0 ? r + n : r;
+    return r >= n ? r - n : r;
+}
+
 // The force fields of consecutive steps, force[step][x, y][node]: a workgroup forms
 // FF_ROWS rows of 256 columns of one step.  TABLE: 2 the table copied to LDS, 1 read
-// from memory, 0 none.
+// from memory, 0 none.  Bound by its vector instructions, seven per node and mode: phases
+// are byte offsets into the table, the rows' formed once per workgroup by as many threads
+// as there are (mode, row) pairs (22.3 us with an integer product per node and mode and a
+// division per mode; entries spread over the LDS banks cost 2 us more than they save).
 constexpr int FF_NT = 256, FF_ROWS = 8, FF_LDS = 2048;
 template <int TABLE>
 __global__ __launch_bounds__(FF_NT) void k_force_field(const ForceTable* __restrict__ tab,
@@ -739,7 +751,8 @@ __global__ __launch_bounds__(FF_NT) void k_force_field(const ForceTable* __restr
                                                        float* __restrict__ force, int nx, int ny) {
     __shared__ float4 mode[MAX_FORCE_MODES];  // sine and cosine coefficients, x and y amplitudes
     __shared__ int kxs[MAX_FORCE_MODES];
-    __shared__ int rowk[MAX_FORCE_MODES][FF_ROWS];  // the rows' phases, in units of 1 / ny
+    // the rows' phases, in units of 1 / ny or as byte offsets into the table
+    __shared__ __align__(16) unsigned rowk[MAX_FORCE_MODES][FF_ROWS];
     __shared__ float2 lt[TABLE == 2 ? FF_LDS : 1];
     const int n = tab->n;
     const int y0 = blockIdx.y * FF_ROWS;
@@ -749,25 +762,32 @@ __global__ __launch_bounds__(FF_NT) void k_force_field(const ForceTable* __restr
         const float2 d = draws[(long long)blockIdx.z * MAX_FORCE_MODES + m];
         mode[m] = make_float4(d.x, d.y, tab->amp[m] * two_pi * float(ky), tab->amp[m] * two_pi * float(-kx));
         kxs[m] = kx;
-        for (int r = 0; r < FF_ROWS; ++r) rowk[m][r] = phase_step(ky, y0 + r, ny);
+    }
+    const long long lx = L / nx, ly = L / ny;
+    for (int k = threadIdx.x; k < n * FF_ROWS; k += FF_NT) {
+        const int m = k / FF_ROWS, r = k % FF_ROWS;
+        rowk[m][r] = unsigned(phase_step(int(tab->ky[m]), y0 + r, ny)) * (TABLE > 0 ? unsigned(8 * ly) : 1u);
     }
     if (TABLE == 2)
         for (int k = threadIdx.x; k < L; k += FF_NT) lt[k] = table[k];
     __syncthreads();
     const int i = blockIdx.x * FF_NT + threadIdx.x;
     if (i >= nx) return;
-    const long long lx = L / nx, ly = L / ny;
+    const float inv_nx = 1.f / float(nx);
     float fx[FF_ROWS] = {}, fy[FF_ROWS] = {};
     for (int m = 0; m < n; ++m) {
         const float4 w = mode[m];
-        const long long col = phase_step(kxs[m], i, nx) * lx;
+        const int kx = __builtin_amdgcn_readfirstlane(kxs[m]);
+        const int c = nx <= (1 << 14) && abs(kx) <= 256 ? phase_small(kx, i, nx, inv_nx) : phase_step(kx, i, nx);
+        const long long col = c * lx;
 #pragma unroll
         for (int r = 0; r < FF_ROWS; ++r) {
             float2 sc;
             if (TABLE > 0) {
-                int k = int(col) + rowk[m][r] * int(ly);
-                k = k >= int(L) ? k - int(L) : k;
-                sc = TABLE == 2 ? lt[k] : table[k];
+                unsigned k = 8u * unsigned(col) + rowk[m][r];
+                k = min(k, k - 8u * unsigned(L));  // wraps to above where k < L
+                sc = *reinterpret_cast<const float2*>(
+                    reinterpret_cast<const char*>(TABLE == 2 ? lt : table) + k);
             } else {
                 const long long k = col + rowk[m][r] * ly;
                 sc = phase_sincos(k >= L ? k - L : k, L);

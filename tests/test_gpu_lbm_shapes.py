@@ -23,6 +23,7 @@ STEPS = 11  # whole launches of two, three and four steps, each with a remainder
     (128, 96, 64),    # three-step strips, a tuned height
     (600, 40, 24),    # two-step strips
     (1031, 1021, 1),  # forcing phases past the table
+    (16500, 8, 1),    # forcing phases of a row past their FP32 quotient
 ])
 def test_default_shape(lb, orc, nx, ny, M, forced):
     cfg = lb.preset("ref" if forced else "baseline")
