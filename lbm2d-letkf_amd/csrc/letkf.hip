@@ -313,7 +313,8 @@ __global__ __launch_bounds__(GRAM_NT) void k_gram_fp32(
 // are gathered in the order member(c) = 4 (c % 4) + c / 4: row and column j of the FP64
 // matrix are then both member(j).  left[g]: what the eigensolve still has to do (a local
 // problem of condition above 65500, or a dumped gridpoint).
-// Bound by the FP64 matrix cores: 96^2 x 64 takes 0.66 ms, against 1.34 ms for C and
+// Bound by the FP64 matrix cores: 96^2 x 64 takes 0.59 ms (0.68 ms with the tiles below
+// the diagonals computed, and 40 bytes of each lane spilled), against 1.34 ms for C and
 // 64.8 ms for the eigensolve in LDS.
 // ----------------------------------------------------------------------------
 struct SeriesParams {
@@ -331,6 +332,7 @@ k_series_fp64(const int* __restrict__ loc_ptr, const int* __restrict__ loc_site,
               const double4* __restrict__ table, int* __restrict__ status, unsigned char* __restrict__ left) {
     constexpr int NT = N / 16;
     __shared__ __align__(16) f64x4 basis[4 * NT * 64];
+    __shared__ double mirror[NT > 1 ? MIRROR64_TILE : 1];
     const int nb = gridDim.x;  // a multiple of 8: each XCD takes a contiguous range
     const int g = int(blockIdx.x % 8) * (nb / 8) + int(blockIdx.x / 8);
     if (g >= p.nodes) return;
@@ -372,7 +374,7 @@ k_series_fp64(const int* __restrict__ loc_ptr, const int* __restrict__ loc_site,
             for (int I = 0; I < NT; ++I) {
                 const float wa = w[s] * xr[s][I];
 #pragma unroll
-                for (int J = 0; J < NT; ++J)
+                for (int J = I; J < NT; ++J)
                     acc[I * NT + J] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa, xc[s][J], acc[I * NT + J], 0, 0, 0);
                 acc[NT * NT + I] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa, c == 9 ? yo[s] : 0.f, acc[NT * NT + I], 0, 0, 0);
             }
@@ -393,9 +395,11 @@ k_series_fp64(const int* __restrict__ loc_ptr, const int* __restrict__ loc_site,
     }
     SeriesMat64<N> m;
 #pragma unroll
-    for (int t = 0; t < NT * NT; ++t)
+    for (int I = 0; I < NT; ++I)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) m.t[t][k] = double(acc[t][k]);
+        for (int J = I; J < NT; ++J)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) m.t[I * NT + J][k] = double(acc[I * NT + J][k]);
     // variable c of members 16 T + 4 grp + k; b in column 9
     const float* fq = f + (long long)(c < Q ? c : 0) * p.nodes + g;
     f64x4 r[NT];
@@ -418,7 +422,7 @@ k_series_fp64(const int* __restrict__ loc_ptr, const int* __restrict__ loc_site,
             const double dx = c < Q && 16 * T + 4 * grp + k < M ? r[T][k] - xbar : 0.0;
             r[T][k] = c == 9 ? double(acc[NT * NT + T][k]) : dx;
         }
-    const int steps = series_apply64<N>(m, r, double(p.diag), table, basis, lane);
+    const int steps = series_apply64<N>(m, r, double(p.diag), table, basis, mirror, lane);
     if (lane == 0) left[g] = steps == 0;
     if (steps == 0) return;
     double dw = 0;  // dX w, w = C^-1 b in column 9

@@ -445,15 +445,34 @@ __device__ __forceinline__ int series_apply(const f32x4* acc, f32x4 (&r)[N / 16]
 // accumulator tiles are operands as they stand here too.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
+constexpr int MIRROR64_TILE = 16 * 17;
 template <int N>
 struct SeriesMat64 {
     static constexpr int NT = N / 16;
     f64x4 t[NT * NT];  // tile (K, J)
+    // the tiles below the diagonal from those above, transposed through LDS (lane (c, g)
+    // holds rows g + 4 r of column c): 8 LDS instructions a tile against 16 matrix
+    // instructions of 64 cycles in a square
+    __device__ __forceinline__ void mirror(double* lds, int lane) {
+        const int c = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = i + 1; j < NT; ++j) {
+                wave_lds_fence();  // (the reads before)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) lds[c * 17 + g + 4 * r] = t[i * NT + j][r];
+                wave_lds_fence();
+#pragma unroll
+                for (int r = 0; r < 4; ++r) t[j * NT + i][r] = lds[(g + 4 * r) * 17 + c];
+            }
+    }
+    // d = this * this, the tiles on and above the diagonal
     __device__ __forceinline__ void square(f64x4 (&d)[NT * NT]) const {
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) d[i * NT + j] = f64x4{0, 0, 0, 0};
+            for (int j = i; j < NT; ++j) d[i * NT + j] = f64x4{0, 0, 0, 0};
 #pragma unroll
         for (int K = 0; K < NT; ++K)
 #pragma unroll
@@ -461,7 +480,7 @@ struct SeriesMat64 {
 #pragma unroll
                 for (int i = 0; i < NT; ++i)
 #pragma unroll
-                    for (int j = 0; j < NT; ++j)
+                    for (int j = i; j < NT; ++j)
                         d[i * NT + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(t[K * NT + i][r], t[K * NT + j][r],
                                                                              d[i * NT + j], 0, 0, 0);
     }
@@ -479,11 +498,13 @@ struct SeriesMat64 {
     }
 };
 
-// r := f(C) r, as series_apply; m holds A and is overwritten; basis: 4 N 16 doubles of
-// LDS, basis[(j NT + T) 64 + lane] the incoming r (j = 0) afterwards.
+// r := f(C) r, as series_apply; m holds A in its tiles on and above the diagonal and is
+// overwritten; basis: 4 N 16 doubles of LDS, basis[(j NT + T) 64 + lane] the incoming r
+// (j = 0) afterwards; mirror: MIRROR64_TILE doubles of LDS.
 template <int N>
 __device__ __forceinline__ int series_apply64(SeriesMat64<N>& m, f64x4 (&r)[N / 16], double a,
-                                              const double4* __restrict__ table, f64x4* basis, int lane) {
+                                              const double4* __restrict__ table, f64x4* basis, double* mirror,
+                                              int lane) {
     constexpr int NT = N / 16;
     auto put = [&](int j, const f64x4 (&x)[NT]) {
 #pragma unroll
@@ -493,13 +514,22 @@ __device__ __forceinline__ int series_apply64(SeriesMat64<N>& m, f64x4 (&r)[N / 
     const double ia = 1.0 / a;
     f64x4 sq[NT * NT];
 #pragma unroll
-    for (int t = 0; t < NT * NT; ++t) m.t[t] *= ia;  // spectrum [0, kappa - 1]
+    for (int I = 0; I < NT; ++I)
+#pragma unroll
+        for (int J = I; J < NT; ++J) m.t[I * NT + J] *= ia;  // spectrum [0, kappa - 1]
+    m.mirror(mirror, lane);
     m.square(sq);
-    double ss = 0;
+    double ss = 0, st = 0;
 #pragma unroll
-    for (int t = 0; t < NT * NT; ++t)
+    for (int I = 0; I < NT; ++I)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) ss = fma(sq[t][k], sq[t][k], ss);
+        for (int J = I; J < NT; ++J)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const double x = sq[I * NT + J][k];
+                (I == J ? ss : st) = fma(x, x, I == J ? ss : st);
+            }
+    ss += 2.0 * st;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
     const float kappa = 1.f + 1.0001f * float(sqrt(sqrt(ss)));
@@ -534,19 +564,21 @@ __device__ __forceinline__ int series_apply64(SeriesMat64<N>& m, f64x4 (&r)[N / 
 #pragma unroll
     for (int I = 0; I < NT; ++I)
 #pragma unroll
-        for (int J = 0; J < NT; ++J)
+        for (int J = I; J < NT; ++J)
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 m.t[I * NT + J][k] = fma(k2, sq[I * NT + J][k],
                                          fma(k1, m.t[I * NT + J][k], I == J && g + 4 * k == c ? 1.0 : 0.0));
+    m.mirror(mirror, lane);
     m.square(sq);
 #pragma unroll
     for (int I = 0; I < NT; ++I)
 #pragma unroll
-        for (int J = 0; J < NT; ++J)
+        for (int J = I; J < NT; ++J)
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 m.t[I * NT + J][k] = fma(4.0, sq[I * NT + J][k], I == J && g + 4 * k == c ? -2.0 : 0.0);
+    m.mirror(mirror, lane);
     const double4* coef = table + first + (c == 9 ? 1 : 0);
     f64x4 b1[NT], b2[NT];
     {
