@@ -557,8 +557,8 @@ int analysis_launches(Ctx* c) {
     HIP_TRY(c, launch_obs_prepare(*c));
     prof_end(c, PH_OBS, e0, 2, n_obs);
     if (c->cfg.variant == LBMLETKF_VARIANT_MIXED && mixed_fused(*c)) {
-        // k_mixed_analysis: gather, MFMA Gram, FP32 sweeps, assembly and update in
-        // one kernel, without workspace
+        // k_series_analysis: gather, MFMA Gram, series and update; then k_mixed_analysis,
+        // the same with FP32 sweeps, for what it left
         hipEvent_t e2 = prof_begin(c);
         HIP_TRY(c, launch_letkf_mixed(*c, c->f[c->cur], c->prof ? c->d_sweeps : nullptr, nullptr,
                                       c->cfg.gram_passes, nullptr, nullptr));

@@ -2,7 +2,7 @@
 sweeps (above) on both sides of the line and with both in one analysis, at member counts
 at the edges of the 16-member tiles, against the FP64 oracle.
 
-The tolerance is the mixed variant's (the split-bf16 Gram matrix sets the error)."""
+The tolerance is the mixed variant's (the sweeps' split-bf16 Gram matrix sets it)."""
 import numpy as np
 import pytest
 
